@@ -49,8 +49,11 @@ struct Handle {
   FrontArgs fr{};
   std::vector<int32_t> fr_lv_ptr, fr_lv_maxm;  // host copies for the launches
   // fronts of more than fr.big_m rows by level (host, offsets, device)
-  std::vector<int32_t> fr_big, fr_big_ptr;
-  int32_t *fr_big_dev = nullptr;
+  std::vector<BigFront> fr_big;
+  std::vector<int32_t> fr_big_ptr;
+  BigFront *fr_big_dev = nullptr;
+  int32_t fr_mv_n = 0;    // large fronts that fr.mv has room for
+  int64_t fr_lbuf_n = 0;  // doubles in fr.lbuf
   std::vector<int64_t> fr_xr_off;  // receiving rows per front (host copy)
   int32_t *d_rowptr = nullptr, *d_colidx = nullptr;
   int32_t *slot_comp = nullptr;
@@ -497,7 +500,6 @@ int xg_lu_solve(xg_handle *H, const double *J, const double *rhs, double *x,
     f.big = h.fr_big_dev;
     f.big_host = h.fr_big.data();
     f.big_ptr_host = h.fr_big_ptr.data();
-    f.xr_off_host = h.fr_xr_off.data();
     e = xg::launch_fronts(f, u, h.stream);
     if (e != hipSuccess) return hip_fail(e, "front LU");
   }
@@ -554,13 +556,37 @@ static int front_big_lists(xg::Handle &h) {
   const xg::LuPlan &L = h.plan.lu;
   h.fr_big.clear();
   h.fr_big_ptr.assign(1, 0);
+  int32_t most = 0;     // of a level
+  int64_t most_lo = 0;  // panel buffers of a level
   for (size_t l = 0; l + 1 < L.fr_lv_ptr.size(); ++l) {
+    int64_t lo = 0;
     for (int32_t q = L.fr_lv_ptr[l]; q < L.fr_lv_ptr[l + 1]; ++q)
-      if (L.fr_m[L.fr_lv[q]] > h.fr.big_m) h.fr_big.push_back(L.fr_lv[q]);
+      if (L.fr_m[L.fr_lv[q]] > h.fr.big_m) {
+        const int32_t s = L.fr_lv[q];
+        const bool have = !h.fr_xr_off.empty();
+        h.fr_big.push_back({L.fr_fo[s], L.fr_ro[s], have ? h.fr_xr_off[s] : 0,
+                            have ? h.fr_xr_off[s + 1] : 0, lo, L.fr_m[s], L.fr_k[s],
+                            L.fr_comp[s], s});
+        lo += (int64_t)xg::kBigW * L.fr_m[s];
+      }
+    most_lo = std::max(most_lo, lo);
+    most = std::max(most, (int32_t)h.fr_big.size() - h.fr_big_ptr.back());
     h.fr_big_ptr.push_back((int32_t)h.fr_big.size());
   }
+  most = std::min(most, (int32_t)xg::kBigLaunch);
+  // (earlier, smaller buffers live on: a captured graph may hold them)
+  if (h.fr_big_dev && most > h.fr_mv_n) {
+    h.fr.mv = h.alloc<int32_t>((size_t)most * xg::kMoveInts);
+    if (!h.fr.mv) return XG_E_NOMEM;
+    h.fr_mv_n = most;
+  }
+  if (h.fr_big_dev && most_lo > h.fr_lbuf_n) {
+    h.fr.lbuf = h.alloc<double>((size_t)most_lo);
+    if (!h.fr.lbuf) return XG_E_NOMEM;
+    h.fr_lbuf_n = most_lo;
+  }
   if (h.fr_big_dev && !h.fr_big.empty() &&
-      hipMemcpy(h.fr_big_dev, h.fr_big.data(), sizeof(int32_t) * h.fr_big.size(),
+      hipMemcpy(h.fr_big_dev, h.fr_big.data(), sizeof(xg::BigFront) * h.fr_big.size(),
                 hipMemcpyHostToDevice) != hipSuccess)
     return XG_E_HIP;
   return XG_OK;
@@ -967,8 +993,14 @@ static bool upload_handle(xg_handle *H) {
       chk(f.v = h.alloc<double>((size_t)(P.n_nodes > 0 ? P.n_nodes : 1)));
       chk(f.piv = h.alloc<int32_t>((size_t)L.fr_ro.back()));
       chk(f.bad = h.alloc<int32_t>((size_t)(u.n_comp > 0 ? u.n_comp : 1)));
-      chk(h.fr_big_dev = h.alloc<int32_t>((size_t)f.n_fronts));
-      if (ok && front_big_lists(h)) ok = false;
+      f.n_rows = L.fr_ro.back();
+      {
+        std::vector<int32_t> rsrc(L.fr_rows.size(), -1);
+        for (int32_t s = 0; s < f.n_fronts; ++s)
+          for (int32_t i = 0; i < L.fr_k[s]; ++i)
+            rsrc[(size_t)(L.fr_ro[s] + i)] = L.fr_rows[(size_t)(L.fr_ro[s] + i)];
+        chk(f.rsrc = h.upload(rsrc));
+      }
       // the children's contribution rows grouped by the row they land on
       // (children in order within each row), for the many-workgroup form
       {
@@ -1005,7 +1037,8 @@ static bool upload_handle(xg_handle *H) {
           xr_off[s + 1] = (int64_t)xr_row.size();
         }
         h.fr_xr_off = xr_off;
-        chk(f.xr_off = h.upload(xr_off));
+        chk(h.fr_big_dev = h.alloc<xg::BigFront>((size_t)nf));
+        if (ok && front_big_lists(h)) ok = false;
         chk(f.xr_row = h.upload(xr_row));
         chk(f.ext_ptr = h.upload(ext_ptr));
         chk(f.ext_ch = h.upload(ext_ch));

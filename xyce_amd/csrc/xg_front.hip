@@ -8,17 +8,19 @@
 // and has m >= k rows; its m x m block is row-major in one value buffer.
 // Per Newton iteration:
 //  1. every front is cleared and the Jacobian's entries are scattered into
-//     the fronts that own them;
+//     the fronts that own them; the right-hand side is one more column of
+//     each front (its fully summed rows' entries, zero below);
 //  2. level by level from the leaves (a level's fronts are independent),
-//     one workgroup per front adds its children's contribution blocks (in
-//     child order), then factors its k fully summed columns: blocked
-//     right-looking LU, pivots chosen by magnitude among the fully summed
-//     rows only, panels in LDS, the trailing update leaving the Schur
-//     complement (the contribution block) in the bottom-right corner;
-//  3. the forward solve runs the same levels: a front gathers its
-//     right-hand side, adds its children's remainders, applies its row
-//     swaps, solves with its unit lower block and leaves the remainder for
-//     its parent; the backward solve walks the levels back down;
+//     a front adds its children's contribution blocks (in child order), then
+//     factors its k fully summed columns: blocked right-looking LU, pivots
+//     chosen by magnitude among the fully summed rows only, the trailing
+//     update leaving the Schur complement (the contribution block) in the
+//     bottom-right corner.  The right-hand-side column takes the same swaps
+//     and updates, so the forward solve is done when the factorisation is,
+//     and L is not kept;
+//  3. the backward solve walks the levels back down;
+// The updates are fused multiply-adds in ascending pivot order in every
+// form below, so all forms give an element the same bits.
 //  4. one workgroup per component checks the normwise backward error
 //     against the unfactored rows, applies x += dx and forms the weighted
 //     RMS norm, as the task-list kernel does.
@@ -83,28 +85,41 @@ __device__ __forceinline__ double blk_reduce(double v, double *sv, bool is_max) 
   return r;
 }
 
-// Partial LU of the m x m row-major front A: its first k columns, pivots
-// among rows [j, k) for column j.  Panels of NB columns factor in the LDS
-// buffer P (rows kb..m-1, stride NB + 1); the panel's row swaps are then
-// applied to the other columns, U12 is solved column by column in
-// registers and the trailing block takes the panel's rank-NB update (each
-// element's updates in ascending pivot order, as in the column-by-column
-// algorithm).  piv[j] = the row swapped with row j.  False when a pivot
-// column has no nonzero candidate.
-//
-// Columns [k0, k1) only, with the row swaps applied to columns [swap_lo, cl)
-// and the updates confined to columns below cl: one panel of the
-// many-workgroup form below, which applies the swaps left of swap_lo
-// afterwards (k0 = 0, k1 = k, cl = m, swap_lo = 0 is the whole
-// factorization).
+// Division by a pivot shared by many rows: the pivot's mantissa p, its
+// reciprocal r and minus its exponent, then per row a quotient and one
+// correction with the exact remainder (four operations instead of the ~11 of
+// a full division; the last bit's error is that of one rounding but for
+// rare double roundings).  Scaling by the exponent keeps the whole range.
+// Every form below divides this way, so all give the same bits.
+struct Pivot {
+  double p, r;
+  int e;
+};
+__device__ __forceinline__ Pivot make_pivot(double v) {
+  const double p = __builtin_amdgcn_frexp_mant(v);
+  return {p, 1.0 / p, -__builtin_amdgcn_frexp_exp(v)};
+}
+__device__ __forceinline__ double divide(double a, const Pivot &v) {
+  const double x = __builtin_amdgcn_ldexp(a, v.e);
+  const double q = x * v.r;
+  return fma(fma(-q, v.p, x), v.r, q);
+}
+
+// Partial LU of the m x m row-major front A and its right-hand side w (the
+// virtual column m): its first k columns, pivots among rows [j, k) for
+// column j.  Panels of NB columns factor in the LDS buffer P (rows
+// kb..m-1, stride NB + 1); the panel's row swaps are then applied to the
+// columns right of it, U12 is solved column by column in registers and the
+// trailing block takes the panel's rank-NB update (each element's updates
+// in ascending pivot order, as in the column-by-column algorithm).  False
+// when a pivot column has no nonzero candidate.
 template <int NB, int BS = kFB>
-__device__ bool front_factor(double *A, int m, int k, double *P, double *sv, int *si,
-                             int *spiv, int32_t *piv, int k0, int k1, int cl,
-                             int swap_lo = 0) {
+__device__ bool front_factor(double *A, double *w, int m, int k, double *P, double *sv,
+                             int *si, int *spiv) {
   const int t = threadIdx.x;
   constexpr int PS = NB + 1;
-  for (int kb = k0; kb < k1; kb += NB) {
-    const int nb = min(NB, k1 - kb);
+  for (int kb = 0; kb < k; kb += NB) {
+    const int nb = min(NB, k - kb);
     const int rows = m - kb;      // panel rows
     const int cand = k - kb;      // rows eligible as pivots
     for (int e = t; e < rows * NB; e += BS) {
@@ -134,51 +149,57 @@ __device__ bool front_factor(double *A, int m, int k, double *P, double *sv, int
           P[br * PS + cc] = tmp;
         }
       __syncthreads();
-      const double pv = P[c * PS + c];
+      const Pivot pv = make_pivot(P[c * PS + c]);
       for (int r = c + 1 + t; r < rows; r += BS) {
-        const double l = P[r * PS + c] / pv;
+        const double l = divide(P[r * PS + c], pv);
         P[r * PS + c] = l;
-        for (int cc = c + 1; cc < nb; ++cc) P[r * PS + cc] -= l * P[c * PS + cc];
+        for (int cc = c + 1; cc < nb; ++cc)
+          P[r * PS + cc] = fma(-l, P[c * PS + cc], P[r * PS + cc]);
       }
       __syncthreads();
     }
-    for (int e = t; e < rows * NB; e += BS) {
+    for (int e = t; e < nb * NB; e += BS) {  // U11 (and L11, unused later)
       const int r = e / NB, c = e % NB;
       if (c < nb) A[(int64_t)(kb + r) * m + kb + c] = P[r * PS + c];
     }
-    if (t < nb) piv[kb + t] = spiv[t];
-    // the panel's row swaps on every other column, in pivot order
-    for (int j = swap_lo + t; j < cl; j += BS) {
-      if (j >= kb && j < kb + nb) continue;
+    const int j0 = kb + nb, ncols = m + 1 - j0;
+    // column j of the front, j = m the right-hand side
+    auto col = [&](int j, int64_t &ld) {
+      ld = j < m ? m : 1;
+      return j < m ? A + j : w;
+    };
+    // the panel's row swaps on the columns right of it, in pivot order
+    for (int j = j0 + t; j <= m; j += BS) {
+      int64_t ld;
+      double *a = col(j, ld);
       for (int c = 0; c < nb; ++c) {
         const int pr = spiv[c];
         if (pr != kb + c) {
-          const double tmp = A[(int64_t)(kb + c) * m + j];
-          A[(int64_t)(kb + c) * m + j] = A[(int64_t)pr * m + j];
-          A[(int64_t)pr * m + j] = tmp;
+          const double tmp = a[(kb + c) * ld];
+          a[(kb + c) * ld] = a[pr * ld];
+          a[pr * ld] = tmp;
         }
       }
     }
     __syncthreads();
-    const int j0 = kb + nb, ncols = cl - j0;
     // U12 of column j (rows kb..kb+nb-1) by the unit lower panel block
-    auto solve_u = [&](int j, double *u) {
+    auto solve_u = [&](const double *a, int64_t ld, double *u) {
 #pragma unroll
-      for (int c = 0; c < NB; ++c) u[c] = c < nb ? A[(int64_t)(kb + c) * m + j] : 0.0;
+      for (int c = 0; c < NB; ++c) u[c] = c < nb ? a[(kb + c) * ld] : 0.0;
 #pragma unroll
       for (int c = 0; c < NB; ++c)
 #pragma unroll
         for (int i = c + 1; i < NB; ++i)
-          if (i < nb) u[i] -= P[i * PS + c] * u[c];
+          if (i < nb) u[i] = fma(-P[i * PS + c], u[c], u[i]);
     };
-    // rows j0+g, j0+g+G, ... of column j take the panel's updates
-    auto sweep = [&](int j, int g, int G, const double *u) {
+    // rows j0+g, j0+g+G, ... of a column take the panel's updates
+    auto sweep = [&](double *a, int64_t ld, int g, int G, const double *u) {
       for (int i = j0 + g; i < m; i += 4 * G) {
         double x[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int ii = i + q * G;
-          x[q] = ii < m ? A[(int64_t)ii * m + j] : 0.0;
+          x[q] = ii < m ? a[ii * ld] : 0.0;
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -187,34 +208,39 @@ __device__ bool front_factor(double *A, int m, int k, double *P, double *sv, int
             const double *l = P + (ii - kb) * PS;
             double v = x[q];
 #pragma unroll
-            for (int c = 0; c < NB; ++c) v -= l[c] * u[c];
-            A[(int64_t)ii * m + j] = v;
+            for (int c = 0; c < NB; ++c)
+              if (c < nb) v = fma(-l[c], u[c], v);
+            a[ii * ld] = v;
           }
         }
       }
     };
     if (ncols >= BS) {
-      for (int j = j0 + t; j < cl; j += BS) {
+      for (int j = j0 + t; j <= m; j += BS) {
+        int64_t ld;
+        double *a = col(j, ld);
         double u[NB];
-        solve_u(j, u);
+        solve_u(a, ld, u);
 #pragma unroll
         for (int c = 0; c < NB; ++c)
-          if (c < nb) A[(int64_t)(kb + c) * m + j] = u[c];
-        sweep(j, 0, 1, u);
+          if (c < nb) a[(kb + c) * ld] = u[c];
+        sweep(a, ld, 0, 1, u);
       }
-    } else if (ncols > 0) {
+    } else {
       const int G = min(BS / ncols, 16);
       const bool mine = t < ncols * G;
-      const int j = j0 + t % ncols, g = t / ncols;
+      const int g = t / ncols;
+      int64_t ld;
+      double *a = col(j0 + t % ncols, ld);
       double u[NB];
-      if (mine) solve_u(j, u);
+      if (mine) solve_u(a, ld, u);
       __syncthreads();
       if (mine) {
         if (g == 0)
 #pragma unroll
           for (int c = 0; c < NB; ++c)
-            if (c < nb) A[(int64_t)(kb + c) * m + j] = u[c];
-        sweep(j, g, G, u);
+            if (c < nb) a[(kb + c) * ld] = u[c];
+        sweep(a, ld, g, G, u);
       }
     }
     __syncthreads();
@@ -226,13 +252,25 @@ __device__ __forceinline__ bool front_skip(const FrontArgs &f, int c) {
   return (f.gate && *f.gate) || (f.active && !f.active[c]) || f.bad[c];
 }
 
-// Clears the fronts and the failure flags, then (second kernel) scatters
-// the Jacobian's entries into them.
-__global__ void __launch_bounds__(kFB) front_clear_kernel(FrontArgs f) {
+// p[i], or 0 where it may not be read (p[0] may): a select, no branch, so
+// that a run of these loads is in flight together (behind `cond ? p[i] : 0`
+// with a short-circuit the compiler waits for each one).
+__device__ __forceinline__ double load_if(bool ok, const double *p, int64_t i) {
+  const double v = p[ok ? i : 0];
+  return ok ? v : 0.0;
+}
+
+// Clears the fronts and the failure flags and sets the right-hand-side
+// columns, then (second kernel) scatters the Jacobian's entries.
+__global__ void __launch_bounds__(kFB) front_clear_kernel(FrontArgs f, const double *bp) {
   if (f.gate && *f.gate) return;
   const int64_t stride = (int64_t)gridDim.x * kFB;
   for (int64_t i = (int64_t)blockIdx.x * kFB + threadIdx.x; i < f.n_vals; i += stride)
     f.vals[i] = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kFB + threadIdx.x; i < f.n_rows; i += stride) {
+    const int32_t r = f.rsrc[i];
+    f.wrhs[i] = r >= 0 ? bp[r] : 0.0;
+  }
   for (int64_t i = (int64_t)blockIdx.x * kFB + threadIdx.x; i < f.n_comp; i += stride)
     f.bad[i] = 0;
 }
@@ -256,20 +294,22 @@ __global__ void __launch_bounds__(BS) front_factor_kernel(FrontArgs f, int lv0) 
   const int t = threadIdx.x;
   const int m = f.m[s], k = f.k[s];
   if (m > f.big_m) return;  // factored by many workgroups (launch_big_front)
-  double *A = f.vals + f.fo[s];
+  double *A = f.vals + f.fo[s], *w = f.wrhs + f.ro[s];
   // the children's contribution blocks, in child order
   for (int q = f.ch_ptr[s]; q < f.ch_ptr[s + 1]; ++q) {
     const int ch = f.ch[q];
-    const int mc = f.m[ch], kc = f.k[ch], w = mc - kc;
+    const int mc = f.m[ch], kc = f.k[ch], wc = mc - kc;
     const double *C = f.vals + f.fo[ch] + (int64_t)kc * mc + kc;
+    const double *r = f.wrhs + f.ro[ch] + kc;
     const int32_t *map = f.cbmap + f.ro[ch] + kc;
-    for (int64_t e = t; e < (int64_t)w * w; e += BS) {
-      const int i = (int)(e / w), j = (int)(e % w);
+    for (int64_t e = t; e < (int64_t)wc * wc; e += BS) {
+      const int i = (int)(e / wc), j = (int)(e % wc);
       A[(int64_t)map[i] * m + map[j]] += C[(int64_t)i * mc + j];
     }
+    for (int i = t; i < wc; i += BS) w[map[i]] += r[i];
     __syncthreads();
   }
-  if (!front_factor<NB, BS>(A, m, k, P, sv, si, spiv, f.piv + f.ro[s], 0, k, m))
+  if (!front_factor<NB, BS>(A, w, m, k, P, sv, si, spiv))
     if (t == 0) f.bad[c] = 1;
 }
 
@@ -289,16 +329,18 @@ __global__ void __launch_bounds__(64) front_tiny_kernel(FrontArgs f, int lv0, in
   if (front_skip(f, c)) return;
   const int m = f.m[s], k = f.k[s];
   if (m > f.big_m) return;
-  double *A = f.vals + f.fo[s];
+  double *A = f.vals + f.fo[s], *w = f.wrhs + f.ro[s];
   for (int qq = f.ch_ptr[s]; qq < f.ch_ptr[s + 1]; ++qq) {
     const int ch = f.ch[qq];
-    const int mc = f.m[ch], kc = f.k[ch], w = mc - kc;
+    const int mc = f.m[ch], kc = f.k[ch], wc = mc - kc;
     const double *C = f.vals + f.fo[ch] + (int64_t)kc * mc + kc;
+    const double *r = f.wrhs + f.ro[ch] + kc;
     const int32_t *map = f.cbmap + f.ro[ch] + kc;
-    for (int i = 0; i < w; ++i)
-      for (int j = 0; j < w; ++j) A[map[i] * m + map[j]] += C[i * mc + j];
+    for (int i = 0; i < wc; ++i) {
+      for (int j = 0; j < wc; ++j) A[map[i] * m + map[j]] += C[i * mc + j];
+      w[map[i]] += r[i];
+    }
   }
-  int32_t *piv = f.piv + f.ro[s];
   for (int col = 0; col < k; ++col) {
     double best = -1.0;
     int br = col;
@@ -313,254 +355,525 @@ __global__ void __launch_bounds__(64) front_tiny_kernel(FrontArgs f, int lv0, in
       f.bad[c] = 1;
       return;
     }
-    piv[col] = br;
-    if (br != col)
-      for (int j = 0; j < m; ++j) {
+    if (br != col) {
+      for (int j = col; j < m; ++j) {
         const double tmp = A[col * m + j];
         A[col * m + j] = A[br * m + j];
         A[br * m + j] = tmp;
       }
-    const double pv = A[col * m + col];
+      const double tmp = w[col];
+      w[col] = w[br];
+      w[br] = tmp;
+    }
+    const Pivot pv = make_pivot(A[col * m + col]);
+    const double wp = w[col];
     for (int r = col + 1; r < m; ++r) {
-      const double l = A[r * m + col] / pv;
-      A[r * m + col] = l;
-      for (int j = col + 1; j < m; ++j) A[r * m + j] -= l * A[col * m + j];
+      const double l = divide(A[r * m + col], pv);
+      for (int j = col + 1; j < m; ++j) A[r * m + j] = fma(-l, A[col * m + j], A[r * m + j]);
+      w[r] = fma(-l, wp, w[r]);
     }
   }
 }
 
 // ---- many-workgroup form of the large fronts (rows m > big_m), all of a
 // level's at once (blockIdx.y or .z = the front among the level's large
-// ones, f.big[lb + that]): per panel of kBigW fully summed columns, one
-// workgroup per front factors the panel (swaps on the columns left of the
-// panel's end), then the columns right of it take the panel's row swaps
-// and their U12 rows (one thread per column), then the trailing block
-// takes the rank-kBigW update in 64 x 64 tiles.  A front whose columns
-// are all factored leaves the later panel launches at once.  Every element
-// sees the same operations in the same order as in the one-workgroup
-// form, so both give the same bits.
-constexpr int kBigW = 32;   // panel width
-// threads of a panel workgroup (per logic factorisation, 256: 5.8 ms of
-// panels, 512: 4.2 ms, 1024: 5.9 ms)
-constexpr int kPanelBlock = 512;
+// ones, f.big[lb + that]).  Per panel of up to kBigW fully summed columns:
+//  panel    one workgroup per front factors the panel's fully summed rows
+//           (the only pivot candidates);
+//  solve    the columns right of it, the right-hand side included, take the
+//           panel's row swaps and their U12 rows (a lane per column), and
+//           the rows below the fully summed block their L21 (a lane per
+//           row): one launch, 64-lane workgroups;
+//  update   the trailing block takes the rank-kBigW update, 64 x 64 tiles on
+//           the FP64 matrix cores.
+// A front whose columns are all factored leaves the later launches at once.
 constexpr int kTile = 64;   // trailing-update tile
 
 // The children's contribution blocks, one workgroup per receiving row of
 // a front (blockIdx.x = the row among the front's receiving rows): the
 // child rows that land on it, in child order, each added across its
-// columns, so every element takes its children's terms in child order.
+// columns and the right-hand side, so every element takes its children's
+// terms in child order.
 __global__ void __launch_bounds__(kFB) front_extend_kernel(FrontArgs f, int lb) {
-  const int s = f.big[lb + blockIdx.y];
-  if (front_skip(f, f.comp[s])) return;
-  const int64_t q = f.xr_off[s] + blockIdx.x;
-  if (q >= f.xr_off[s + 1]) return;
-  const int m = f.m[s];
-  double *Ar = f.vals + f.fo[s] + (int64_t)f.xr_row[q] * m;
+  const BigFront s = f.big[lb + blockIdx.y];
+  if (front_skip(f, s.comp)) return;
+  const int64_t q = s.xr0 + blockIdx.x;
+  if (q >= s.xr1) return;
+  const int m = s.m;
+  const int row = f.xr_row[q];
+  double *Ar = f.vals + s.fo + (int64_t)row * m;
+  double *wr = f.wrhs + s.ro + row;
   for (int64_t e = f.ext_ptr[q]; e < f.ext_ptr[q + 1]; ++e) {
     const int ch = f.ext_ch[e], i = f.ext_i[e];
     const int mc = f.m[ch], kc = f.k[ch], w = mc - kc;
     const double *C = f.vals + f.fo[ch] + (int64_t)(kc + i) * mc + kc;
     const int32_t *map = f.cbmap + f.ro[ch] + kc;
     for (int j = threadIdx.x; j < w; j += kFB) Ar[map[j]] += C[j];
+    if (threadIdx.x == 0) *wr += f.wrhs[f.ro[ch] + kc + i];
     __syncthreads();
   }
 }
 
-template <int NB, int ROWS, int BS>
-__global__ void __launch_bounds__(BS) front_panel_kernel(FrontArgs f, int lb, int kb) {
-  __shared__ double P[ROWS * (NB + 1)];
-  __shared__ double sv[BS / 64];
-  __shared__ int si[BS / 64];
-  __shared__ int spiv[NB];
-  const int s = f.big[lb + blockIdx.x];
-  const int c = f.comp[s];
-  if (front_skip(f, c)) return;
-  const int m = f.m[s], k = f.k[s];
-  if (kb >= k) return;
-  const int cl = min(kb + kBigW, k);
-  if (!front_factor<NB, BS>(f.vals + f.fo[s], m, k, P, sv, si, spiv, f.piv + f.ro[s], kb, cl,
-                            cl, kb))
-    if (threadIdx.x == 0) f.bad[c] = 1;
+// Maximum of a word over lanes 0 .. 63 (kSteps = 6) or 0 .. 2^kSteps - 1, from
+// that range's last lane: row shifts, then the row broadcasts, each folded
+// into one v_max_u32.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ unsigned dpp_max(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, false);
+  return o > v ? o : v;
 }
-
-// Columns j >= cl: the panel's row swaps in pivot order, then U12 = L11^-1
-// (rows kb..cl-1) with the unit lower panel block, each u[i] updated in
-// ascending pivot order.
-// One wavefront per 64 columns: the work is a few dependent loads and a
-// 32-term solve per column, so more, smaller workgroups spread it over
-// more CUs.
-constexpr int kSwapBlock = 64;
-
-__global__ void __launch_bounds__(kSwapBlock) front_swap_trsm_kernel(FrontArgs f, int lb, int kb) {
-  __shared__ double L11[kBigW][kBigW + 1];
-  __shared__ int32_t pv[kBigW];
-  const int s = f.big[lb + blockIdx.y];
-  if (front_skip(f, f.comp[s])) return;
-  const int m = f.m[s], k = f.k[s];
-  if (kb >= k) return;
-  const int cl = min(kb + kBigW, k), nw = cl - kb;
-  if (cl + (int)(blockIdx.x * kSwapBlock) >= m) return;
-  double *A = f.vals + f.fo[s];
-  const int32_t *piv = f.piv + f.ro[s];
-  for (int e = threadIdx.x; e < kBigW * kBigW; e += kSwapBlock) {
-    const int i = e / kBigW, cc = e % kBigW;
-    L11[i][cc] = (i < nw && cc < nw) ? A[(int64_t)(kb + i) * m + kb + cc] : 0.0;
-  }
-  if (threadIdx.x < kBigW) pv[threadIdx.x] = threadIdx.x < nw ? piv[kb + threadIdx.x] : 0;
-  __syncthreads();
-  const int j = cl + blockIdx.x * kSwapBlock + threadIdx.x;
-  if (j >= m) return;
-  for (int cc = 0; cc < nw; ++cc) {
-    const int pr = pv[cc];
-    if (pr != kb + cc) {
-      const double tmp = A[(int64_t)(kb + cc) * m + j];
-      A[(int64_t)(kb + cc) * m + j] = A[(int64_t)pr * m + j];
-      A[(int64_t)pr * m + j] = tmp;
+template <int kSteps>
+__device__ __forceinline__ unsigned lanes_max(unsigned v) {
+  if (kSteps > 0) v = dpp_max<0x111, 0xf>(v);
+  if (kSteps > 1) v = dpp_max<0x112, 0xf>(v);
+  if (kSteps > 2) v = dpp_max<0x114, 0xf>(v);
+  if (kSteps > 3) v = dpp_max<0x118, 0xf>(v);
+  if (kSteps > 4) v = dpp_max<0x142, 0xa>(v);
+  if (kSteps > 5) v = dpp_max<0x143, 0xc>(v);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, (1 << kSteps) - 1);
+}
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// The lane (of the first 2^kSteps) with the largest v >= 0, the smallest p
+// on ties (lanes holding no candidate: v = 0, which never wins over one).
+// Magnitudes order as their bits do: the high words first, the low ones
+// only where several high words tie.
+template <int kSteps>
+__device__ __forceinline__ int lane_of_max(double v, int p) {
+  constexpr unsigned long long kLanes = kSteps > 5 ? ~0ull : (1ull << (1 << kSteps)) - 1;
+  const unsigned hi = (unsigned)__double2hiint(v), lo = (unsigned)__double2loint(v);
+  const unsigned mh = lanes_max<kSteps>(hi);
+  unsigned long long mask = __ballot(hi == mh) & kLanes;
+  if (mask & (mask - 1)) {
+    const unsigned ml = lanes_max<kSteps>(hi == mh ? lo : 0u);
+    mask = __ballot(hi == mh && lo == ml) & kLanes;
+    if (mh | ml) {
+      int lane = __ffsll(mask) - 1;
+      int best = __builtin_amdgcn_readlane(p, lane);
+      for (mask &= mask - 1; mask; mask &= mask - 1) {
+        const int b = __ffsll(mask) - 1;
+        const int o = __builtin_amdgcn_readlane(p, b);
+        if (o < best) {
+          best = o;
+          lane = b;
+        }
+      }
+      return lane;
     }
   }
-  double u[kBigW];
-#pragma unroll
-  for (int cc = 0; cc < kBigW; ++cc) u[cc] = cc < nw ? A[(int64_t)(kb + cc) * m + j] : 0.0;
-#pragma unroll
-  for (int cc = 0; cc < kBigW; ++cc)
-#pragma unroll
-    for (int i = cc + 1; i < kBigW; ++i)
-      if (i < nw) u[i] -= L11[i][cc] * u[cc];
-#pragma unroll
-  for (int cc = 0; cc < kBigW; ++cc)
-    if (cc < nw) A[(int64_t)(kb + cc) * m + j] = u[cc];
+  return __ffsll(mask) - 1;
 }
 
-// Rows and columns >= cl: A -= L21 U12, each element's terms in ascending
-// pivot order.  Grid: (tiles over columns, tiles over rows, fronts).
-__global__ void __launch_bounds__(kFB) front_update_kernel(FrontArgs f, int lb, int kb) {
-  __shared__ double Lt[kTile][kBigW + 1];
-  __shared__ double Ut[kBigW][kTile + 1];
-  const int s = f.big[lb + blockIdx.z];
-  if (front_skip(f, f.comp[s])) return;
-  const int m = f.m[s], k = f.k[s];
+// One panel: columns [kb, kb + W) of the rows [kb, k), W = 16 kCT.  The panel
+// stays in registers as 16 x 16 tiles in the layout of the FP64 matrix cores
+// (below), kNT tiles of rows per wavefront.  Four columns at a time go
+// through LDS to one row per lane (kNT / 4 rows), where a column step is:
+// the largest candidate of the wavefront by DPP, each wavefront's candidate
+// row of four to LDS, one barrier, then every lane takes the best one and
+// updates its rows' four columns.  The remaining columns then take the four
+// pivot rows' U (solved by every lane for its column) and one rank-4 product
+// per tile.  Rows are not moved: a lane tracks the position its row has
+// after the swaps (ties go to the smallest position, as in the other forms).
+// Finished pivot rows go to their position of A; the multipliers go to the
+// column-major panel buffer by original row, with f.piv the original row of
+// each position and f.mv the rows displaced from the panel's block.
+// What bounds it is a column step's chain (~700 cycles: two searches of 200,
+// the exchange through LDS of 300, the division).  With whole rows of 32 in
+// lanes the exchange of a row (32 b128 LDS operations of ~40 cycles each)
+// took 4000 cycles a column.
+typedef double double4v __attribute__((ext_vector_type(4)));
+
+template <int NW, int kNT, int kCT>
+__global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int lb, int kb) {
+  constexpr int R = kNT / 4, W = 16 * kCT, kRows = 16 * kNT;
+  static_assert(kNT % 4 == 0 && (NW == 1 || NW == 4 || NW == 8), "rows per lane, search");
+  __shared__ __align__(16) double S[NW][kRows][4];
+  __shared__ __align__(16) double srow[2][4][NW][4];
+  __shared__ double sval[2][4][NW], srcp[2][4][NW], raw[4][W];
+  __shared__ int spos[2][4][NW], sphy[2][4][NW], nmove;
+  const BigFront s = f.big[lb + blockIdx.x];
+  if (front_skip(f, s.comp)) return;
+  const int m = s.m, k = s.k;
   if (kb >= k) return;
-  const int cl = min(kb + kBigW, k), nw = cl - kb;
-  double *A = f.vals + f.fo[s];
+  const int nw = min(W, k - kb), nr = k - kb;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int wrow = wave * kRows;
+  double *A = f.vals + s.fo + (int64_t)kb * m + kb;
+  double *L = f.lbuf + s.lo + kb;  // column c: L + c m
+  if (threadIdx.x == 0) nmove = 0;
+  double4v acc[kNT][kCT];
+#pragma unroll
+  for (int t = 0; t < kNT; ++t)
+#pragma unroll
+    for (int c = 0; c < kCT; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = wrow + 16 * t + lk + 4 * r, j = 16 * c + li;
+        acc[t][c][r] = load_if((i < nr) & (j < nw), A, (int64_t)i * m + j);
+      }
+  int pos[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int r = wrow + 64 * q + lane;
+    pos[q] = r < nr ? r : -1;
+  }
+#pragma unroll
+  for (int ct = 0; ct < kCT; ++ct) {
+#pragma unroll 1
+    for (int s4 = 0; s4 < 4; ++s4) {  // (one copy: the code must stay in the cache)
+      const int c0 = 16 * ct + 4 * s4;
+      if (c0 >= nw) break;
+      const int par = s4 & 1;
+      // four columns to one row per lane
+      if ((li >> 2) == s4)
+#pragma unroll
+        for (int t = 0; t < kNT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[wave][16 * t + lk + 4 * r][li & 3] = acc[t][ct][r];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      double a[R][4], ln[R][4];
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          a[q][j] = S[wave][64 * q + lane][j];
+          ln[q][j] = -0.0;
+        }
+      unsigned win = 0;  // the wavefront of each pivot row, four bits each
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = c0 + j;
+        if (c >= nw) continue;
+        double v = 0.0, x0 = 0.0;
+        int p = 0x7fffffff, qb = 0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const double x = fabs(a[q][j]);
+          if (pos[q] >= c && (x > v || (x == v && pos[q] < p))) {
+            v = x;
+            x0 = a[q][j];
+            p = pos[q];
+            qb = q;
+          }
+        }
+        // the reciprocal every lane's candidate would need, while the
+        // search below waits on its chain
+        double rcp = make_pivot(x0).r;
+        const int wl = lane_of_max<6>(v, p);
+        if (lane == wl) {
+          sval[par][j][wave] = v;
+          srcp[par][j][wave] = rcp;
+          spos[par][j][wave] = p;
+          sphy[par][j][wave] = wrow + 64 * qb + lane;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            double x = a[0][jj];
+#pragma unroll
+            for (int q = 1; q < R; ++q) {
+              double aq = a[q][jj];
+              asm("" : "+v"(aq));  // a select of values, not an indexed load
+              x = qb == q ? aq : x;
+            }
+            srow[par][j][wave][jj] = x;
+          }
+        }
+        int bw = 0;
+        double best;
+        if constexpr (NW == 1) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          best = sval[par][j][0];
+        } else {
+          __syncthreads();
+          // the best wavefront: lanes 0..NW-1 hold the candidates
+          const double cv = lane < NW ? sval[par][j][lane] : 0.0;
+          const int cp = lane < NW ? spos[par][j][lane] : 0x7fffffff;
+          bw = lane_of_max<NW == 8 ? 3 : 2>(cv, cp);
+          best = read_lane(cv, bw);
+        }
+        if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
+          if (threadIdx.x == 0) f.bad[s.comp] = 1;
+          return;
+        }
+        win |= (unsigned)bw << (4 * j);
+        const int bp = spos[par][j][bw];
+        double u[4];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) u[jj] = srow[par][j][bw][jj];
+        const Pivot pv{__builtin_amdgcn_frexp_mant(u[j]), srcp[par][j][bw],
+                       -__builtin_amdgcn_frexp_exp(u[j])};
+        // the finished pivot row's entries of these columns
+        if (wave == 0 && lane >= j && lane < 4 && c0 + lane < nw)
+          A[(int64_t)c * m + c0 + lane] = srow[par][j][bw][lane];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          pos[q] = pos[q] == bp ? c : (pos[q] == c ? bp : pos[q]);
+          if (pos[q] > c) {
+            const double l = divide(a[q][j], pv);
+            L[(int64_t)c * m + wrow + 64 * q + lane] = l;
+            a[q][j] = l;
+            ln[q][j] = -l;
+#pragma unroll
+            for (int jj = j + 1; jj < 4; ++jj) a[q][jj] = fma(-l, u[jj], a[q][jj]);
+          }
+        }
+      }
+      if (c0 + 4 >= nw) break;
+      // the four pivot rows' other columns, from the lanes that hold them
+#pragma unroll 1
+      for (int j = 0; j < 4; ++j) {
+        const int ph =
+            __builtin_amdgcn_readfirstlane(sphy[par][j][win >> (4 * j) & 15]) - wrow;
+        if (ph < 0 || ph >= kRows) continue;
+#pragma unroll
+        for (int t = 0; t < kNT; ++t)
+          if ((ph >> 4) == t) {
+            const int r = (ph >> 2) & 3;
+#pragma unroll
+            for (int q = ct; q < kCT; ++q) {
+              const double4v x = acc[t][q];
+              const double y = r == 0 ? x[0] : r == 1 ? x[1] : r == 2 ? x[2] : x[3];
+              if (lk == (ph & 3)) raw[j][16 * q + li] = y;
+            }
+            asm volatile("; tile %0" ::"n"(t));  // (kept apart: fixed registers)
+          }
+      }
+      if constexpr (NW == 1) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      } else {
+        __syncthreads();
+      }
+      double ub[kCT];
+#pragma unroll
+      for (int q = ct; q < kCT; ++q) {
+        double u[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          u[j] = raw[j][16 * q + li];
+#pragma unroll
+          for (int i = 0; i < j; ++i) u[j] = fma(-srow[par][j][win >> (4 * j) & 15][i], u[i], u[j]);
+        }
+        const int col = 16 * q + li;
+        const double x = lk == 0 ? u[0] : lk == 1 ? u[1] : lk == 2 ? u[2] : u[3];
+        ub[q] = col >= c0 + 4 ? x : 0.0;
+        if (wave == 0 && col >= c0 + 4 && col < nw) A[(int64_t)(c0 + lk) * m + col] = x;
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[wave][64 * q + lane][j] = ln[q][j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int t = 0; t < kNT; ++t) {
+        const double av = S[wave][16 * t + li][lk];
+#pragma unroll
+        for (int q = ct; q < kCT; ++q)
+          acc[t][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, ub[q], acc[t][q], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  int32_t *piv = f.piv + s.ro + kb;
+  int32_t *mv = f.mv + (int64_t)blockIdx.x * kMoveInts;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int r = wrow + 64 * q + lane;
+    if (pos[q] >= 0) {
+      piv[pos[q]] = kb + r;
+      if (pos[q] >= nw && pos[q] != r) {
+        const int e = atomicAdd(&nmove, 1);  // at most nw rows
+        mv[1 + 2 * e] = kb + pos[q];
+        mv[2 + 2 * e] = kb + r;
+      }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) mv[0] = nmove;
+}
+
+// After a panel.  Workgroups [0, column blocks): a lane per column j >= cl
+// (j = m the right-hand side): the rows the swaps bring into the panel's
+// block and the block's rows they displace, all loaded at once, then U12 =
+// L11^-1 (each u[i] updated in ascending pivot order).  The others: a lane
+// per row >= k, L21 = A21 U11^-1 through a transposing LDS tile (each entry
+// updated in ascending pivot order, then divided by its pivot, as the
+// right-looking form does), to the panel buffer.  One swap at a time, each
+// waiting for the last one's stores, took 40 us per panel of the 5,000-gate
+// logic.
+__global__ void __launch_bounds__(64) front_solve_kernel(FrontArgs f, int lb, int kb, int wp) {
+  __shared__ double D[kBigW][kBigW + 1];
+  __shared__ double T[64][kBigW + 1];
+  __shared__ double dr[kBigW];
+  __shared__ int32_t top[kBigW], mdst[kBigW], msrc[kBigW];
+  const BigFront s = f.big[lb + blockIdx.y];
+  if (front_skip(f, s.comp)) return;
+  const int m = s.m, k = s.k;
+  if (kb >= k) return;
+  const int cl = min(kb + wp, k), nw = cl - kb;
+  const int ncb = (m + 1 - cl + 63) / 64, nrb = (m - k + 63) / 64;
+  const int lane = threadIdx.x;
+  const int b = blockIdx.x;
+  if (b >= ncb + nrb) return;
+  double *A = f.vals + s.fo;
+  double *L = f.lbuf + s.lo;
+  constexpr int RI = 64 / kBigW;
+  const int lr = lane / kBigW, lc = lane % kBigW;
+  if (b < ncb) {
+    const int32_t *mv = f.mv + (int64_t)blockIdx.y * kMoveInts;
+    const int nm = mv[0];
+    if (lane < kBigW) {  // (padded with readable rows, so no load below is conditional)
+      top[lane] = lane < nw ? f.piv[s.ro + kb + lane] : kb;
+      mdst[lane] = lane < nm ? mv[1 + 2 * lane] : kb;
+      msrc[lane] = lane < nm ? mv[2 + 2 * lane] : kb;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kBigW / RI; ++i) {  // L11, columns in rows of D
+      const int c = i * RI + lr;
+      D[c][lc] = load_if((c < lc) & (lc < nw), L, (int64_t)c * m + top[lc]);
+    }
+    const int j = cl + b * 64 + lane, jc = min(j, m);
+    double *col = jc < m ? A + jc : f.wrhs + s.ro;
+    const int ld = jc < m ? m : 1;
+    double u[kBigW], d[kBigW];
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c) u[c] = col[top[c] * ld];
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c) d[c] = col[msrc[c] * ld];
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c) asm("" : "+v"(d[c]));  // (not sunk to their stores)
+    __syncthreads();
+    if (j > m) return;
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c)
+      if (c < nm) col[mdst[c] * ld] = d[c];
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c) {
+      if (c < nw)
+#pragma unroll
+        for (int i = c + 1; i < kBigW; ++i) u[i] = fma(-D[c][i], u[c], u[i]);
+      __builtin_amdgcn_sched_barrier(0);  // D's reads stay by their column
+    }
+#pragma unroll
+    for (int c = 0; c < kBigW; ++c)
+      if (c < nw) col[(kb + c) * ld] = u[c];
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < kBigW / RI; ++i) {
+    const int r = i * RI + lr;
+    D[r][lc] = load_if((r <= lc) & (lc < nw), A, (int64_t)(kb + r) * m + kb + lc);
+  }
+  const int r0 = k + (b - ncb) * 64;
+#pragma unroll
+  for (int i = 0; i < 64 / RI; ++i) {
+    const int r = min(r0 + i * RI + lr, m - 1);
+    T[i * RI + lr][lc] = A[(int64_t)r * m + kb + min(lc, nw - 1)];
+  }
+  __syncthreads();
+  if (lane < kBigW) dr[lane] = make_pivot(D[lane][lane]).r;
+  __syncthreads();
+  double l[kBigW];
+#pragma unroll
+  for (int c = 0; c < kBigW; ++c) l[c] = T[lane][c];
+#pragma unroll
+  for (int c = 0; c < kBigW; ++c) {
+    if (c < nw) {
+      const double d = D[c][c];
+      l[c] = divide(l[c], {__builtin_amdgcn_frexp_mant(d), dr[c], -__builtin_amdgcn_frexp_exp(d)});
+#pragma unroll
+      for (int i = c + 1; i < kBigW; ++i) l[i] = fma(-l[c], D[c][i], l[i]);
+      if (r0 + lane < m) L[(int64_t)c * m + r0 + lane] = l[c];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Rows and columns >= cl: A -= L21 U12, and the right-hand side's rows.
+// Grid: (tiles over columns, tiles over rows, fronts).  Each wavefront takes
+// a 32 x 32 quarter of the tile as 2 x 2 products of 16 x 16 x 4
+// (v_mfma_f64_16x16x4: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
+// D[l / 16 + 4 r][l % 16]; its result is the fused multiply-adds in
+// ascending k, so these are the bits of the scalar form).  One element per
+// thread with two LDS reads per multiply-add took 21 us per panel of the
+// 5,000-gate logic.
+__global__ void __launch_bounds__(kFB) front_update_kernel(FrontArgs f, int lb, int kb,
+                                                           int wp) {
+  __shared__ double Lt[kBigW][kTile + 1];  // -L21, columns in rows
+  __shared__ double Ut[kBigW][kTile + 1];
+  __shared__ double y[kBigW];
+  const BigFront s = f.big[lb + blockIdx.z];
+  if (front_skip(f, s.comp)) return;
+  const int m = s.m, k = s.k;
+  if (kb >= k) return;
+  const int cl = min(kb + wp, k), nw = cl - kb;
+  double *A = f.vals + s.fo, *w = f.wrhs + s.ro;
   const int r0 = cl + blockIdx.y * kTile, c0 = cl + blockIdx.x * kTile;
   if (r0 >= m || c0 >= m) return;
-  for (int e = threadIdx.x; e < kTile * kBigW; e += kFB) {
-    const int r = e / kBigW, cc = e % kBigW;
-    Lt[r][cc] = (r0 + r < m && cc < nw) ? A[(int64_t)(r0 + r) * m + kb + cc] : 0.0;
-  }
-  for (int e = threadIdx.x; e < kBigW * kTile; e += kFB) {
-    const int cc = e / kTile, q = e % kTile;
-    Ut[cc][q] = (cc < nw && c0 + q < m) ? A[(int64_t)(kb + cc) * m + c0 + q] : 0.0;
-  }
-  __syncthreads();
-  // thread: one column of the tile, rows r, r + 4, ... (16 rows)
-  const int q = threadIdx.x % kTile, rg = threadIdx.x / kTile;
-  const int j = c0 + q;
-  if (j >= m) return;
-  for (int r = rg; r < kTile; r += kFB / kTile) {
-    const int i = r0 + r;
-    if (i >= m) break;
-    double v = A[(int64_t)i * m + j];
-    for (int cc = 0; cc < nw; ++cc) v -= Lt[r][cc] * Ut[cc][q];
-    A[(int64_t)i * m + j] = v;
-  }
-}
-
-// The row swaps of the later panels on the factored columns j < k (the L
-// part), deferred from the panels: column j takes every pivot after its
-// own panel, in pivot order, as the one-workgroup form applies them.
-__global__ void __launch_bounds__(kFB) front_left_swaps_kernel(FrontArgs f, int lb) {
-  const int s = f.big[lb + blockIdx.y];
-  if (front_skip(f, f.comp[s])) return;
-  const int m = f.m[s], k = f.k[s];
-  const int j = blockIdx.x * kFB + threadIdx.x;
-  if (j >= k) return;
-  double *A = f.vals + f.fo[s];
-  const int32_t *piv = f.piv + f.ro[s];
-  for (int c = (j / kBigW + 1) * kBigW; c < k; ++c) {
-    const int pr = piv[c];
-    if (pr != c) {
-      const double tmp = A[(int64_t)c * m + j];
-      A[(int64_t)c * m + j] = A[(int64_t)pr * m + j];
-      A[(int64_t)pr * m + j] = tmp;
-    }
-  }
-}
-
-// Forward solve of one level's fronts: the front's right-hand side (its
-// fully summed rows' entries, zero below), its children's remainders,
-// its row swaps, then L y = b with the unit lower columns; y goes to the
-// position vector, the remainder below stays in wrhs for the parent.
-// Blocked by 64 columns: the diagonal block on one wavefront (the
-// solution broadcast by lane shuffles), then every row below takes the
-// block's 64 terms.  Each element takes its terms in ascending column
-// order, as the column-by-column algorithm gives them.
-template <int ROWS, int BS>
-__global__ void __launch_bounds__(BS) front_fwd_kernel(FrontArgs f, const double *bp,
-                                                        int lv0) {
-  __shared__ double ws[ROWS];
-  const int s = f.lv[lv0 + blockIdx.x];
-  const int c = f.comp[s];
-  if (front_skip(f, c)) return;
   const int t = threadIdx.x;
-  const int m = f.m[s], k = f.k[s];
-  const double *A = f.vals + f.fo[s];
-  const int32_t *rows = f.rows + f.ro[s];
-  double *w = f.wrhs + f.ro[s];
-  for (int i = t; i < m; i += BS) ws[i] = i < k ? bp[rows[i]] : 0.0;
-  __syncthreads();
-  for (int q = f.ch_ptr[s]; q < f.ch_ptr[s + 1]; ++q) {
-    const int ch = f.ch[q];
-    const int kc = f.k[ch], wc = f.m[ch] - kc;
-    const double *r = f.wrhs + f.ro[ch] + kc;
-    const int32_t *map = f.cbmap + f.ro[ch] + kc;
-    for (int i = t; i < wc; i += BS) ws[map[i]] += r[i];
-    __syncthreads();
-  }
-  // the row swaps in pivot order: one wavefront finds the pivots that
-  // move a row (64 at a time) and its first lane applies just those
-  const int32_t *pv = f.piv + f.ro[s];
-  if (t < 64) {
-    for (int j0 = 0; j0 < k; j0 += 64) {
-      const int j = j0 + t;
-      const int p = j < k ? pv[j] : j;
-      unsigned long long mv = __ballot(p != j);
-      while (mv) {
-        const int b = __ffsll(mv) - 1;
-        const int pb = __shfl(p, b);
-        if (t == 0) {
-          const double tmp = ws[j0 + b];
-          ws[j0 + b] = ws[pb];
-          ws[pb] = tmp;
-        }
-        mv &= mv - 1;
+  const int wave = t >> 6, lane = t & 63, li = lane & 15, lk = lane >> 4;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  double4v acc[2][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = r0 + wr + 16 * p + lk + 4 * r, j = c0 + wc + 16 * q + li;
+        acc[p][q][r] = load_if((i < m) & (j < m), A, (int64_t)i * m + j);
       }
+  // padding: a product of -0.0, the identity of the sum
+  {
+    // (rows below the fully summed block stay where they are)
+    const int i = r0 + lane;
+    const int src = i < k ? f.piv[s.ro + i] : i;
+    const double *L = f.lbuf + s.lo;
+#pragma unroll
+    for (int q = 0; q < kBigW / 4; ++q) {
+      const int cc = 4 * q + wave;
+      Lt[cc][lane] = -load_if((i < m) & (cc < nw), L, (int64_t)cc * m + src);
     }
   }
+#pragma unroll
+  for (int e = t; e < kBigW * kTile; e += kFB) {
+    const int cc = e / kTile, q = e % kTile;
+    Ut[cc][q] = load_if((cc < nw) & (c0 + q < m), A, (int64_t)(kb + cc) * m + c0 + q);
+  }
+  if (t < kBigW) y[t] = t < nw ? w[kb + t] : 0.0;
   __syncthreads();
-  for (int jb = 0; jb < k; jb += 64) {
-    const int je = min(jb + 64, k);
-    if (t < 64) {
-      const int i = jb + t;
-      double wi = i < je ? ws[i] : 0.0;
-      for (int j = jb; j < je; ++j) {
-        const double yj = __shfl(wi, j - jb);
-        if (i > j && i < je) wi -= A[(int64_t)i * m + j] * yj;
-      }
-      if (i < je) ws[i] = wi;
+  for (int kk = 0; kk < nw; kk += 4) {
+    double av[2], bv[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      av[p] = Lt[kk + lk][wr + 16 * p + li];
+      bv[p] = Ut[kk + lk][wc + 16 * p + li];
     }
-    __syncthreads();
-    for (int i = je + t; i < m; i += BS) {
-      double r = ws[i];
-      const double *a = A + (int64_t)i * m;
-      for (int j = jb; j < je; ++j) r -= a[j] * ws[j];
-      ws[i] = r;
-    }
-    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[p], bv[q], acc[p][q], 0, 0, 0);
   }
-  for (int i = t; i < m; i += BS) {
-    w[i] = ws[i];
-    if (i < k) f.v[rows[i]] = ws[i];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = r0 + wr + 16 * p + lk + 4 * r, j = c0 + wc + 16 * q + li;
+        if (i < m && j < m) A[(int64_t)i * m + j] = acc[p][q][r];
+      }
+  if (blockIdx.x == 0 && t < kTile && r0 + t < m) {
+    double v = w[r0 + t];
+    for (int cc = 0; cc < nw; ++cc) v = fma(Lt[cc][t], y[cc], v);
+    w[r0 + t] = v;
   }
 }
 
@@ -580,6 +893,7 @@ __global__ void __launch_bounds__(BS) front_bwd_kernel(FrontArgs f, int lv0) {
   const int m = f.m[s], k = f.k[s];
   const double *A = f.vals + f.fo[s];
   const int32_t *rows = f.rows + f.ro[s];
+  const double *y = f.wrhs + f.ro[s];
   // the right-hand side less the solved rows below: a wavefront per row,
   // its lanes strided over the row, summed by a fixed shuffle tree
   for (int j = k + t; j < m; j += BS) xs[j - k] = f.v[rows[j]];
@@ -590,7 +904,7 @@ __global__ void __launch_bounds__(BS) front_bwd_kernel(FrontArgs f, int lv0) {
     double p = 0.0;
     for (int j = k + lane; j < m; j += 64) p += a[j] * xs[j - k];
     for (int off = 32; off >= 1; off >>= 1) p += __shfl_xor(p, off);
-    if (lane == 0) tb[i] = f.v[rows[i]] - p;
+    if (lane == 0) tb[i] = y[i] - p;
   }
   __syncthreads();
   for (int jb = ((k - 1) / 64) * 64; jb >= 0 && k > 0; jb -= 64) {
@@ -849,48 +1163,60 @@ hipError_t launch_level(const FrontArgs &f, int lv0, int nfr, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The panel launch for `nr` fully summed rows left, its width: 32 columns
+// while a lane holds at most two rows, so that the tiles fit the registers of
+// eight wavefronts (256 a lane), 16 above.
+int launch_panel(const FrontArgs &f, int lb, int nb, int kb, int nr, hipStream_t s) {
+#define XG_PANEL(NW, NT, CT)                                                             \
+  do {                                                                                   \
+    hipLaunchKernelGGL((front_panel_kernel<NW, NT, CT>), dim3(nb), dim3(64 * NW), 0, s, f, \
+                       lb, kb);                                                          \
+    return 16 * CT;                                                                      \
+  } while (0)
+  if (nr <= 64) XG_PANEL(1, 4, 2);
+  if (nr <= 256) XG_PANEL(4, 4, 2);
+  if (nr <= 512) XG_PANEL(8, 4, 2);
+  if (nr <= 1024) XG_PANEL(8, 8, 2);
+  if (nr <= 2048) XG_PANEL(8, 16, 1);
+  static_assert(kFrontMaxM <= 8 * 16 * 28, "rows of the widest panel form");
+  XG_PANEL(8, 28, 1);
+#undef XG_PANEL
+}
+
 // A level's fronts of more than big_m rows (f.big[lb, lb + nb)) by many
 // workgroups: their children's contribution blocks (one launch, a
-// workgroup per receiving row), then per panel position the panel,
-// swap / U12 and trailing-update launches over all of them, then the
-// deferred left swaps.
+// workgroup per receiving row), then per panel position the panel, solve
+// and trailing-update launches over all of them.
 hipError_t launch_big_fronts(const FrontArgs &f, int lb, int nb, hipStream_t s) {
-  int max_m = 0, max_k = 0;
+  int max_k = 0;
   int64_t max_rows = 0;
   for (int q = lb; q < lb + nb; ++q) {
-    const int sf = f.big_host[q];
-    max_m = std::max(max_m, f.m_host[sf]);
-    max_k = std::max(max_k, f.k_host[sf]);
-    max_rows = std::max(max_rows, f.xr_off_host[sf + 1] - f.xr_off_host[sf]);
+    const BigFront &b = f.big_host[q];
+    max_k = std::max(max_k, b.k);
+    max_rows = std::max(max_rows, b.xr1 - b.xr0);
   }
   if (max_rows > 0)
     hipLaunchKernelGGL(front_extend_kernel, dim3((unsigned)max_rows, nb), dim3(kFB), 0, s, f,
                        lb);
-  for (int kb = 0; kb < max_k; kb += kBigW) {
-    if (max_m <= 1934)
-      hipLaunchKernelGGL((front_panel_kernel<8, 1934, kPanelBlock>), dim3(nb), dim3(kPanelBlock),
-                         0, s, f, lb, kb);
-    else
-      hipLaunchKernelGGL((front_panel_kernel<4, kFrontMaxM, kPanelBlock>), dim3(nb),
-                         dim3(kPanelBlock), 0, s, f, lb,
-                         kb);
-    // the largest trailing block at this panel position
-    int rest = 0;
+  for (int kb = 0; kb < max_k;) {
+    const int wp = launch_panel(f, lb, nb, kb, max_k - kb, s);
+    // the largest trailing block and solve at this panel position
+    int rest = 0, blocks = 0;
     for (int q = lb; q < lb + nb; ++q) {
-      const int sf = f.big_host[q];
-      if (kb < f.k_host[sf])
-        rest = std::max(rest, f.m_host[sf] - std::min(kb + kBigW, f.k_host[sf]));
+      const int m = f.big_host[q].m, k = f.big_host[q].k;
+      if (kb >= k) continue;
+      const int r = m - std::min(kb + wp, k);
+      rest = std::max(rest, r);
+      blocks = std::max(blocks, (r + 1 + 63) / 64 + (m - k + 63) / 64);
     }
-    if (rest <= 0) continue;
-    hipLaunchKernelGGL(front_swap_trsm_kernel, dim3((rest + kSwapBlock - 1) / kSwapBlock, nb),
-                       dim3(kSwapBlock), 0, s, f, lb, kb);
-    const unsigned tiles = (unsigned)((rest + kTile - 1) / kTile);
-    hipLaunchKernelGGL(front_update_kernel, dim3(tiles, tiles, nb), dim3(kFB), 0, s, f, lb,
-                       kb);
+    hipLaunchKernelGGL(front_solve_kernel, dim3(blocks, nb), dim3(64), 0, s, f, lb, kb, wp);
+    if (rest > 0) {
+      const unsigned tiles = (unsigned)((rest + kTile - 1) / kTile);
+      hipLaunchKernelGGL(front_update_kernel, dim3(tiles, tiles, nb), dim3(kFB), 0, s, f, lb,
+                         kb, wp);
+    }
+    kb += wp;
   }
-  if (max_k > kBigW)
-    hipLaunchKernelGGL(front_left_swaps_kernel, dim3((max_k + kFB - 1) / kFB, nb), dim3(kFB),
-                       0, s, f, lb);
   return hipGetLastError();
 }
 
@@ -910,7 +1236,7 @@ hipError_t launch_fronts(const FrontArgs &f, const SparseLuArgs &a, hipStream_t 
   if (f.n_fronts == 0) return hipSuccess;
   const unsigned gclear =
       (unsigned)std::min<int64_t>((std::max(f.n_vals, (int64_t)f.n_comp) + kFB - 1) / kFB, 8192);
-  hipLaunchKernelGGL(front_clear_kernel, dim3(gclear), dim3(kFB), 0, s, f);
+  hipLaunchKernelGGL(front_clear_kernel, dim3(gclear), dim3(kFB), 0, s, f, a.bp);
   const unsigned gsc = (unsigned)std::min<int64_t>((f.n_ent + kFB - 1) / kFB + 1, 8192);
   hipLaunchKernelGGL(front_scatter_kernel, dim3(gsc), dim3(kFB), 0, s, f, a.J);
   hipError_t e = hipGetLastError();
@@ -939,27 +1265,15 @@ hipError_t launch_fronts(const FrontArgs &f, const SparseLuArgs &a, hipStream_t 
       }
       if (e != hipSuccess) return e;
     }
-    // the level's larger fronts, at most 65535 per launch (grid y / z)
+    // the level's larger fronts, at most kBigLaunch per launch (grid y / z)
     if (any_big)
-      for (int lb = f.big_ptr_host[L]; lb < f.big_ptr_host[L + 1]; lb += 65535)
-        if ((e = launch_big_fronts(f, lb, std::min(65535, f.big_ptr_host[L + 1] - lb), s)) !=
+      for (int lb = f.big_ptr_host[L]; lb < f.big_ptr_host[L + 1]; lb += kBigLaunch)
+        if ((e = launch_big_fronts(f, lb, std::min(kBigLaunch, f.big_ptr_host[L + 1] - lb), s)) !=
             hipSuccess)
           return e;
   }
-  // the solves' LDS holds a front's rows: the level's largest front picks
-  // the instance (the largest fronts with 512 threads)
-  for (int L = 0; L < f.n_levels; ++L) {
-    const int lv0 = f.lv_ptr_host[L], nfr = f.lv_ptr_host[L + 1] - lv0;
-    const int mm = f.lv_maxm_host[L];
-    const double *bp = a.bp;
-    if (mm <= 64)
-      hipLaunchKernelGGL((front_fwd_kernel<64, kFB>), dim3(nfr), dim3(kFB), 0, s, f, bp, lv0);
-    else if (mm <= 512)
-      hipLaunchKernelGGL((front_fwd_kernel<512, kFB>), dim3(nfr), dim3(kFB), 0, s, f, bp, lv0);
-    else
-      hipLaunchKernelGGL((front_fwd_kernel<kFrontMaxM, kSolveBlock>), dim3(nfr), dim3(kSolveBlock),
-                         0, s, f, bp, lv0);
-  }
+  // the backward solve's LDS holds a front's rows: the level's largest front
+  // picks the instance (the largest fronts with 512 threads)
   for (int L = f.n_levels - 1; L >= 0; --L) {
     const int lv0 = f.lv_ptr_host[L], nfr = f.lv_ptr_host[L + 1] - lv0;
     const int mm = f.lv_maxm_host[L];

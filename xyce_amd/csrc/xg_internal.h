@@ -280,13 +280,28 @@ struct SparseLuArgs {
 constexpr int kFrontMaxM = 3481;  // largest front a workgroup's panel holds
 // Fronts of more rows are factored by many workgroups per panel.
 constexpr int32_t kFrontBigM = 64;
+constexpr int kBigW = 32;               // most columns of their panels
+constexpr int kMoveInts = 1 + 2 * kBigW;  // FrontArgs::mv per front
+constexpr int kBigLaunch = 65535;       // most large fronts per launch (grid y / z)
+// One large front as its kernels read it (one load instead of a chain).
+struct BigFront {
+  int64_t fo, ro, xr0, xr1;  // values, rows, receiving rows [xr0, xr1)
+  int64_t lo;                // its panel buffer in FrontArgs::lbuf
+  int32_t m, k, comp, id;
+};
 struct FrontArgs {
   int32_t n_fronts = 0, n_comp = 0, n_levels = 0;
-  int64_t n_vals = 0, n_ent = 0;
+  int64_t n_vals = 0, n_ent = 0, n_rows = 0;  // n_rows: front rows, all fronts
   const int32_t *comp, *m, *k, *rows, *cbmap, *ch_ptr, *ch, *lv, *ent_k, *front_comp;
   const int64_t *fo, *ro, *ent_fpos;
+  const int32_t *rsrc;            // at ro[s] + i: rows[i] for i < k[s], else -1
   double *vals, *wrhs, *v;        // fronts, front right-hand sides, positions
-  int32_t *piv, *bad;             // row swaps (at ro), failed components
+  int32_t *piv, *bad;             // panel rows before its swaps (at ro), failed components
+  // per large front of a launch: the rows a panel's swaps displace from its
+  // block, their number, then (dst, src) pairs
+  int32_t *mv = nullptr;
+  // per large front of a level: its panel's multipliers, column c at c m
+  double *lbuf = nullptr;
   const int32_t *active;
   const int32_t *gate = nullptr;  // stop word (LoadPtrs::gate)
   const int32_t *lv_ptr_host, *lv_maxm_host;  // host arrays: the launch loop
@@ -295,15 +310,16 @@ struct FrontArgs {
   const int32_t *lv_host, *m_host, *k_host, *ch_ptr_host, *ch_host;
   int32_t big_m = kFrontBigM;
   // those fronts grouped by level (device), with the host's level offsets
-  const int32_t *big = nullptr, *big_host = nullptr, *big_ptr_host = nullptr;
+  const BigFront *big = nullptr, *big_host = nullptr;
+  const int32_t *big_ptr_host = nullptr;
   // components of more than kFinishSplit unknowns finish in chunks of
   // kFinishChunk rows: per component split[c] (1 = chunked), the chunks'
   // component and first row, the chunked components and their chunk
   // ranges, per-chunk partials (4 doubles) and the per-component verdict
   // children's contribution rows by target: front s's rows that receive
-  // contributions are xr_row[xr_off[s], xr_off[s + 1]); target q takes
+  // contributions are xr_row[xr0, xr1) (BigFront); target q takes
   // child rows (ext_ch, ext_i)[ext_ptr[q], ext_ptr[q + 1]) in child order
-  const int64_t *xr_off = nullptr, *ext_ptr = nullptr, *xr_off_host = nullptr;
+  const int64_t *ext_ptr = nullptr;
   const int32_t *xr_row = nullptr, *ext_ch = nullptr, *ext_i = nullptr;
   // rows of more than kLongRow Jacobian entries (supply rails) per front
   // component, checked by a whole workgroup: long_rows[long_ptr[c], ..)
