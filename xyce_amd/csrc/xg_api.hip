@@ -47,7 +47,7 @@ struct Handle {
   DenseSolveArgs ds{};
   SparseLuArgs lu{};
   FrontArgs fr{};
-  std::vector<int32_t> fr_lv_ptr, fr_lv_maxm;  // host copies for the launches
+  std::vector<int32_t> fr_lv, fr_cls, fr_lv_maxm;  // host copies for the launches
   // fronts of more than fr.big_m rows by level (host, offsets, device)
   std::vector<BigFront> fr_big;
   std::vector<int32_t> fr_big_ptr;
@@ -489,14 +489,11 @@ int xg_lu_solve(xg_handle *H, const double *J, const double *rhs, double *x,
     xg::FrontArgs f = h.fr;
     f.active = active;
     f.gate = h.gate;
-    f.lv_ptr_host = h.fr_lv_ptr.data();
+    f.cls_host = h.fr_cls.data();
     f.lv_maxm_host = h.fr_lv_maxm.data();
     const xg::LuPlan &L = h.plan.lu;
-    f.lv_host = L.fr_lv.data();
+    f.lv_host = h.fr_lv.data();
     f.m_host = L.fr_m.data();
-    f.k_host = L.fr_k.data();
-    f.ch_ptr_host = L.fr_ch_ptr.data();
-    f.ch_host = L.fr_ch.data();
     f.big = h.fr_big_dev;
     f.big_host = h.fr_big.data();
     f.big_ptr_host = h.fr_big_ptr.data();
@@ -970,7 +967,18 @@ static bool upload_handle(xg_handle *H) {
     f.n_fronts = (int32_t)L.fr_m.size();
     f.n_comp = u.n_comp;
     if (f.n_fronts > 0) {
-      h.fr_lv_ptr = L.fr_lv_ptr;
+      // each level's fronts by size class
+      h.fr_lv = L.fr_lv;
+      h.fr_cls.assign(1, 0);
+      for (size_t l = 0; l + 1 < L.fr_lv_ptr.size(); ++l) {
+        const auto b = h.fr_lv.begin() + L.fr_lv_ptr[l], e = h.fr_lv.begin() + L.fr_lv_ptr[l + 1];
+        const auto t = std::stable_partition(
+            b, e, [&](int32_t s) { return L.fr_m[s] <= xg::kTinyM; });
+        const auto g = std::stable_partition(t, e, [&](int32_t s) { return L.fr_m[s] <= 64; });
+        h.fr_cls.push_back((int32_t)(t - h.fr_lv.begin()));
+        h.fr_cls.push_back((int32_t)(g - h.fr_lv.begin()));
+        h.fr_cls.push_back((int32_t)(e - h.fr_lv.begin()));
+      }
       h.fr_lv_maxm = L.fr_lv_maxm;
       f.n_levels = (int32_t)L.fr_lv_maxm.size();
       f.n_vals = L.fr_fo.back();
@@ -982,7 +990,7 @@ static bool upload_handle(xg_handle *H) {
       chk(f.cbmap = h.upload(L.fr_cbmap));
       chk(f.ch_ptr = h.upload(L.fr_ch_ptr));
       chk(f.ch = h.upload(L.fr_ch));
-      chk(f.lv = h.upload(L.fr_lv));
+      chk(f.lv = h.upload(h.fr_lv));
       chk(f.ent_k = h.upload(L.fr_ent_k));
       chk(f.front_comp = h.upload(L.front_comp));
       chk(f.fo = h.upload(L.fr_fo));

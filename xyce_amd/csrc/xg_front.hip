@@ -319,7 +319,6 @@ __global__ void __launch_bounds__(BS) front_factor_kernel(FrontArgs f, int lv0) 
 // the fully summed rows (largest magnitude, smallest index on ties).  Every
 // element takes the same operations in the same order as in the blocked
 // workgroup form, so both give the same bits.
-constexpr int kTinyM = 16;
 
 __global__ void __launch_bounds__(64) front_tiny_kernel(FrontArgs f, int lv0, int nfr) {
   const int q = blockIdx.x * 64 + threadIdx.x;
@@ -697,6 +696,183 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
   if (threadIdx.x == 0) mv[0] = nmove;
 }
 
+// One wavefront per front of up to 64 rows: the front and its right-hand
+// side (column m) in LDS, where the children's contribution blocks are added
+// in child order, then in registers as 16 x 16 tiles, factored like a panel
+// above (four columns at a time to a row per lane, rank-4 matrix-core
+// products of the rest), every column at once.  Same operations per element
+// as the other forms, so the same bits.  A front is a chain of column steps
+// of ~0.5 us; with 16-column panels in LDS and separate passes for swaps, U12
+// and update, 100 x 100 power-grid levels took 62 us on average.
+template <int kNT, int kCT>
+__global__ void __launch_bounds__(64) front_wave_kernel(FrontArgs f, int lv0) {
+  __shared__ double F[16 * kNT][16 * kCT + 1];
+  __shared__ __align__(16) double S[16 * kNT][4], srow[4][4];
+  __shared__ double raw[4][16 * kCT];
+  const int s = f.lv[lv0 + blockIdx.x];
+  const int comp = f.comp[s];
+  if (front_skip(f, comp)) return;
+  const int m = f.m[s], k = f.k[s];
+  if (m > f.big_m) return;  // factored by many workgroups
+  const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+  double *A = f.vals + f.fo[s], *w = f.wrhs + f.ro[s];
+  auto fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  const int row = min(lane, m - 1);
+#pragma unroll 8
+  for (int i = 0; i < m; ++i) {
+    const double v = A[i * m + row];
+    if (lane < m) F[i][lane] = v;
+  }
+  if (lane < m) F[lane][m] = w[lane];
+  fence();
+  for (int q = f.ch_ptr[s]; q < f.ch_ptr[s + 1]; ++q) {
+    const int ch = f.ch[q];
+    const int mc = f.m[ch], kc = f.k[ch], wc = mc - kc;
+    const double *C = f.vals + f.fo[ch] + (int64_t)kc * mc + kc;
+    const int jl = min(lane, max(wc - 1, 0));
+    const int map = wc > 0 ? f.cbmap[f.ro[ch] + kc + jl] : 0;
+    const double r = wc > 0 ? f.wrhs[f.ro[ch] + kc + jl] : 0.0;
+#pragma unroll 8
+    for (int i = 0; i < wc; ++i) {
+      const double v = C[i * mc + jl];
+      const int mi = __builtin_amdgcn_readlane(map, i);
+      if (lane < wc) F[mi][map] += v;
+    }
+    if (lane < wc) F[map][m] += r;
+    fence();
+  }
+  double4v acc[kNT][kCT];
+#pragma unroll
+  for (int t = 0; t < kNT; ++t)
+#pragma unroll
+    for (int c = 0; c < kCT; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][c][r] = F[16 * t + lk + 4 * r][16 * c + li];
+  int pos = lane < k ? lane : lane < m ? lane + 64 : -1;  // (rows >= k: no candidates)
+#pragma unroll 1
+  for (int c0 = 0; c0 < k; c0 += 4) {
+    const int ct = c0 >> 4, nv = min(4, k - c0);
+#pragma unroll
+    for (int q = 0; q < kCT; ++q)
+      if (ct == q) {
+        if ((li >> 2) == ((c0 >> 2) & 3))
+#pragma unroll
+          for (int t = 0; t < kNT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[16 * t + lk + 4 * r][li & 3] = acc[t][q][r];
+        asm volatile("; tile %0" ::"n"(q));  // (kept apart: fixed registers)
+      }
+    fence();
+    double a[4], ln[4];
+    const int sr = min(lane, 16 * kNT - 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[j] = S[sr][j];
+      ln[j] = -0.0;
+    }
+    unsigned win = 0;  // the rows of the four pivots, eight bits each
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = c0 + j;
+      if (j >= nv) continue;
+      const bool cand = pos >= c && pos < k;
+      const double v = cand ? fabs(a[j]) : 0.0;
+      double rcp = make_pivot(a[j]).r;
+      // (a NaN is no candidate, as in the other forms)
+      const int wl = lane_of_max<6>(v > 0.0 ? v : 0.0, cand ? pos : 0x7fffffff);
+      const double best = read_lane(v, wl);
+      const int bp = __builtin_amdgcn_readlane(pos, wl);
+      rcp = read_lane(rcp, wl);
+      if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
+        if (lane == 0) f.bad[comp] = 1;
+        return;
+      }
+      win |= (unsigned)wl << (8 * j);
+      if (lane == wl)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) srow[j][jj] = a[jj];
+      fence();
+      double u[4];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) u[jj] = srow[j][jj];
+      if (lane >= j && lane < nv) A[c * m + c0 + lane] = srow[j][lane];
+      const Pivot pv{__builtin_amdgcn_frexp_mant(u[j]), rcp, -__builtin_amdgcn_frexp_exp(u[j])};
+      pos = pos == bp ? c : (pos == c ? bp : pos);
+      if (pos > c) {
+        const double l = divide(a[j], pv);
+        a[j] = l;
+        ln[j] = -l;
+#pragma unroll
+        for (int jj = j + 1; jj < 4; ++jj) a[jj] = fma(-l, u[jj], a[jj]);
+      }
+    }
+    // the pivot rows' other columns, from the lanes that hold them
+#pragma unroll 1
+    for (int j = 0; j < nv; ++j) {
+      const int ph = win >> (8 * j) & 255;
+#pragma unroll
+      for (int t = 0; t < kNT; ++t)
+        if ((ph >> 4) == t) {
+          const int r = (ph >> 2) & 3;
+#pragma unroll
+          for (int q = 0; q < kCT; ++q) {
+            const double4v x = acc[t][q];
+            const double y = r == 0 ? x[0] : r == 1 ? x[1] : r == 2 ? x[2] : x[3];
+            if (lk == (ph & 3)) raw[j][16 * q + li] = y;
+          }
+          asm volatile("; tile %0" ::"n"(t));
+        }
+    }
+    if (lane < 16 * kNT)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S[lane][j] = ln[j];
+    fence();
+    double av[kNT];
+#pragma unroll
+    for (int t = 0; t < kNT; ++t) av[t] = S[16 * t + li][lk];
+    double l[4][4];
+#pragma unroll
+    for (int j = 1; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < j; ++i) l[j][i] = srow[j][i];
+#pragma unroll
+    for (int q = 0; q < kCT; ++q) {
+      if (q < ct) continue;
+      double u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        u[j] = raw[j][16 * q + li];
+#pragma unroll
+        for (int i = 0; i < j; ++i) u[j] = fma(-l[j][i], u[i], u[j]);
+      }
+      const int col = 16 * q + li;
+      const double x = lk == 0 ? u[0] : lk == 1 ? u[1] : lk == 2 ? u[2] : u[3];
+      const bool on = col >= c0 + nv && lk < nv;
+      if (on && col < m) A[(c0 + lk) * m + col] = x;
+      if (on && col == m) w[c0 + lk] = x;
+      const double ub = on ? x : 0.0;
+#pragma unroll
+      for (int t = 0; t < kNT; ++t)
+        acc[t][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t], ub, acc[t][q], 0, 0, 0);
+    }
+    fence();
+  }
+  // the contribution block and its right-hand side
+#pragma unroll
+  for (int t = 0; t < kNT; ++t)
+#pragma unroll
+    for (int c = 0; c < kCT; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * t + lk + 4 * r, j = 16 * c + li;
+        if (i >= k && i < m && j >= k && j < m) A[i * m + j] = acc[t][c][r];
+        if (i >= k && i < m && j == m) w[i] = acc[t][c][r];
+      }
+}
+
 // After a panel.  Workgroups [0, column blocks): a lane per column j >= cl
 // (j = m the right-hand side): the rows the swaps bring into the panel's
 // block and the block's rows they displace, all loaded at once, then U12 =
@@ -877,62 +1053,140 @@ __global__ void __launch_bounds__(kFB) front_update_kernel(FrontArgs f, int lb, 
   }
 }
 
+// Sum over the 16 lanes of a row, the same bits in every lane: neighbours,
+// then pairs, quads and halves (each step adds two mirror images).
+template <int kCtrl>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return v + __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, 0xf, 0xf, false),
+                              __builtin_amdgcn_update_dpp(lo, lo, kCtrl, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double sum8(double v) {
+  return dpp_add<0x141>(dpp_add<0x4e>(dpp_add<0xb1>(v)));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x140>(sum8(v));
+  return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+}
+
 // Backward solve of one level's fronts (levels from the root down): the
 // rows below the fully summed block are solved already (by ancestors).
-// Blocked by 64 columns from the last: the diagonal block on one
-// wavefront, then every row above takes the block's terms; each element
-// takes its terms in descending column order, as the column-by-column
-// algorithm gives them.
+// First the right-hand side less the solved rows below, a wavefront per
+// row: lane-strided products, summed by wave_sum.  Then blocks of 64 columns
+// from the last: the diagonal block in LDS on the first wavefront, a lane
+// per row, while the others subtract the block solved before it from the
+// rows above (the rows of the next block first, by everyone), eight lanes a
+// row.  The chain of the diagonal blocks (~100 cycles a column: the
+// quotient, its broadcast, the update) and one CU's reads of U are about
+// equal for the largest fronts; with a row per thread and the diagonal read
+// from memory inside the chain a 1540-row front took 1 ms.
 template <int ROWS, int BS>
 __global__ void __launch_bounds__(BS) front_bwd_kernel(FrontArgs f, int lv0) {
-  __shared__ double tb[ROWS], xs[ROWS];
+  constexpr int NW = BS / 64;
+  __shared__ double tb[ROWS], xs[ROWS], D[64][65];
   const int s = f.lv[lv0 + blockIdx.x];
   const int c = f.comp[s];
   if (front_skip(f, c)) return;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   const int m = f.m[s], k = f.k[s];
   const double *A = f.vals + f.fo[s];
   const int32_t *rows = f.rows + f.ro[s];
   const double *y = f.wrhs + f.ro[s];
-  // the right-hand side less the solved rows below: a wavefront per row,
-  // its lanes strided over the row, summed by a fixed shuffle tree
   for (int j = k + t; j < m; j += BS) xs[j - k] = f.v[rows[j]];
   __syncthreads();
-  const int w = t >> 6, lane = t & 63;
-  for (int i = w; i < k; i += BS / 64) {
+  for (int i = w; i < k; i += NW) {
     const double *a = A + (int64_t)i * m;
     double p = 0.0;
-    for (int j = k + lane; j < m; j += 64) p += a[j] * xs[j - k];
-    for (int off = 32; off >= 1; off >>= 1) p += __shfl_xor(p, off);
+#pragma unroll 4
+    for (int j = k + lane; j < m; j += 64) p = fma(a[j], xs[j - k], p);
+    p = wave_sum(p);
     if (lane == 0) tb[i] = y[i] - p;
   }
-  __syncthreads();
-  for (int jb = ((k - 1) / 64) * 64; jb >= 0 && k > 0; jb -= 64) {
-    const int je = min(jb + 64, k);
-    if (t < 64) {
-      const int i = jb + t;
-      double ti = i < je ? tb[i] : 0.0;
-      for (int j = je - 1; j >= jb; --j) {
-        double xj = 0.0;
-        if (i == j) xj = ti / A[(int64_t)j * m + j];
-        xj = __shfl(xj, j - jb);
-        if (i == j)
-          ti = xj;
-        else if (i < j)
-          ti -= A[(int64_t)i * m + j] * xj;
+  // rows [r0, r1) less their columns [c0, c1) times the solved tb there, by
+  // nt threads of which this one is `id`
+  auto subtract = [&](int r0, int r1, int c0, int c1, int id, int nt) {
+    const int sub = id & 7;
+    double x[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = load_if(c0 + 8 * sub + q < c1, tb, c0 + 8 * sub + q);
+#pragma unroll 2
+    for (int r = r0 + (id >> 3); r < r1; r += nt / 8) {
+      const double *a = A + (int64_t)r * m;
+      double v[8], p = 0.0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = load_if(c0 + 8 * sub + q < c1, a, c0 + 8 * sub + q);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) p = fma(v[q], x[q], p);
+      p = sum8(p);
+      if (sub == 0) tb[r] = tb[r] - p;
+    }
+  };
+  for (int jb = ((k - 1) / 64) * 64; jb >= 0; jb -= 64) {
+    const int je = min(jb + 64, k), n = je - jb, je2 = min(je + 64, k);
+    double d[64 * 64 / BS];
+#pragma unroll
+    for (int q = 0; q < 64 * 64 / BS; ++q) {
+      const int e = t + q * BS, r = e >> 6, cc = e & 63;
+      d[q] = load_if((r <= cc) & (cc < n), A, (int64_t)(jb + r) * m + jb + cc);
+    }
+    __syncthreads();  // tb of the block before, and D free
+    if (je < k) subtract(jb, je, je, je2, t, BS);
+#pragma unroll
+    for (int q = 0; q < 64 * 64 / BS; ++q) {
+      const int e = t + q * BS;
+      D[e >> 6][e & 63] = d[q];
+    }
+    __syncthreads();
+    if (w == 0) {
+      double ti = load_if(lane < n, tb, jb + lane);
+      const Pivot pv = make_pivot(lane < n ? D[lane][lane] : 1.0);
+      double dj = D[lane][n - 1];
+      for (int j = n - 1; j >= 0; --j) {
+        const double dn = D[lane][max(j - 1, 0)];
+        const double xj = read_lane(divide(ti, pv), j);
+        ti = lane < j ? fma(-dj, xj, ti) : lane == j ? xj : ti;
+        dj = dn;
       }
-      if (i < je) tb[i] = ti;
+      if (lane < n) tb[jb + lane] = ti;
+    } else if (je < k) {
+      subtract(0, jb, je, je2, t - 64, BS - 64);
     }
-    __syncthreads();
-    for (int i = t; i < jb; i += BS) {
-      double r = tb[i];
-      const double *a = A + (int64_t)i * m;
-      for (int j = je - 1; j >= jb; --j) r -= a[j] * tb[j];
-      tb[i] = r;
-    }
-    __syncthreads();
   }
+  __syncthreads();
   for (int i = t; i < k; i += BS) f.v[rows[i]] = tb[i];
+}
+
+// The same for fronts of up to kTinyM rows, one thread each, with the same
+// operations per element (the products summed as wave_sum sums them).
+__global__ void __launch_bounds__(64) front_tiny_bwd_kernel(FrontArgs f, int lv0, int nfr) {
+  const int q = blockIdx.x * 64 + threadIdx.x;
+  if (q >= nfr) return;
+  const int s = f.lv[lv0 + q];
+  const int c = f.comp[s];
+  if (front_skip(f, c)) return;
+  const int m = f.m[s], k = f.k[s];
+  const double *A = f.vals + f.fo[s];
+  const int32_t *rows = f.rows + f.ro[s];
+  double *y = f.wrhs + f.ro[s];
+  double x[kTinyM];
+#pragma unroll
+  for (int j = 0; j < kTinyM; ++j) x[j] = load_if(k + j < m, f.v, rows[min(k + j, m - 1)]);
+  for (int i = 0; i < k; ++i) {
+    double p[kTinyM];
+#pragma unroll
+    for (int j = 0; j < kTinyM; ++j) p[j] = fma(load_if(k + j < m, A, i * m + k + j), x[j], 0.0);
+#pragma unroll
+    for (int st = 1; st < kTinyM; st *= 2)
+#pragma unroll
+      for (int j = 0; j < kTinyM; j += 2 * st) p[j] = p[j] + p[j + st];
+    // (wave_sum's empty lanes: at least one zero more in every step)
+    y[i] = y[i] - (((p[0] + 0.0) + 0.0) + 0.0);
+  }
+  for (int j = k - 1; j >= 0; --j) {
+    const double xj = divide(y[j], make_pivot(A[j * m + j]));
+    f.v[rows[j]] = xj;
+    for (int i = 0; i < j; ++i) y[i] = fma(-A[i * m + j], xj, y[i]);
+  }
 }
 
 // The residual and |J| row-sum maxima of a component's long rows in
@@ -1149,17 +1403,16 @@ __global__ void __launch_bounds__(64) finish_sum_kernel(FrontArgs f, SparseLuArg
   stats[3] = (double)n;
 }
 
-// One workgroup per front of the level: one wavefront for fronts of up
-// to 64 rows (cheap barriers, four times the workgroups per CU), four for
-// larger ones.  The block size changes which thread does an operation,
-// never an element's operations or their order.
+// Most fronts of up to 64 rows in a level for each to take a wavefront, the
+// ones of up to kTinyM rows included (in place of a launch of their own, a
+// thread each).
+constexpr int kWaveFronts = 2048;
+
+// One workgroup per front of the level (fronts above 64 rows, when the
+// many-workgroup threshold is raised).
 template <int NB, int ROWS>
 hipError_t launch_level(const FrontArgs &f, int lv0, int nfr, hipStream_t s) {
-  if (ROWS <= 64)
-    hipLaunchKernelGGL((front_factor_kernel<NB, ROWS, 64>), dim3(nfr), dim3(64), 0, s, f, lv0);
-  else
-    hipLaunchKernelGGL((front_factor_kernel<NB, ROWS, kFB>), dim3(nfr), dim3(kFB), 0, s, f,
-                       lv0);
+  hipLaunchKernelGGL((front_factor_kernel<NB, ROWS, kFB>), dim3(nfr), dim3(kFB), 0, s, f, lv0);
   return hipGetLastError();
 }
 
@@ -1242,48 +1495,67 @@ hipError_t launch_fronts(const FrontArgs &f, const SparseLuArgs &a, hipStream_t 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   for (int L = 0; L < f.n_levels; ++L) {
-    const int lv0 = f.lv_ptr_host[L], nfr = f.lv_ptr_host[L + 1] - lv0;
-    // the level's fronts up to big_m rows, one workgroup each
-    int32_t small_max = 0;
-    bool any_big = false;
-    for (int q = lv0; q < lv0 + nfr; ++q) {
-      const int32_t mq = f.m_host[f.lv_host[q]];
-      if (mq > f.big_m) any_big = true;
-      else small_max = std::max(small_max, mq);
+    // the level's fronts by size class (kTinyM rows, 64 rows, larger): the
+    // first by threads, the others up to big_m rows by a workgroup each
+    const int32_t *cp = f.cls_host + 3 * L;
+    const int lv0 = cp[0], mid0 = cp[1], big0 = cp[2], lv1 = cp[3];
+    int32_t one_max = 0;  // largest of the last class up to big_m rows
+    for (int q = big0; q < lv1; ++q)
+      if (f.m_host[f.lv_host[q]] <= f.big_m)
+        one_max = std::max(one_max, f.m_host[f.lv_host[q]]);
+    // (a level of few fronts: a wavefront for each of those up to 64 rows)
+    const int wave0 = big0 - lv0 <= kWaveFronts ? lv0 : mid0;
+    if (wave0 > lv0)
+      hipLaunchKernelGGL(front_tiny_kernel, dim3((wave0 - lv0 + 63) / 64), dim3(64), 0, s, f,
+                         lv0, wave0 - lv0);
+    if (big0 > wave0) {
+      int32_t mx = 0;
+      for (int q = wave0; q < big0; ++q) mx = std::max(mx, f.m_host[f.lv_host[q]]);
+#define XG_WAVE(NT, CT) \
+  hipLaunchKernelGGL((front_wave_kernel<NT, CT>), dim3(big0 - wave0), dim3(64), 0, s, f, wave0)
+      if (mx <= 15) XG_WAVE(1, 1);
+      else if (mx <= 31) XG_WAVE(2, 2);
+      else if (mx <= 47) XG_WAVE(3, 3);
+      else if (mx <= 63) XG_WAVE(4, 4);
+      else XG_WAVE(4, 5);
+#undef XG_WAVE
     }
-    if (small_max > 0 && small_max <= kTinyM) {
-      hipLaunchKernelGGL(front_tiny_kernel, dim3((nfr + 63) / 64), dim3(64), 0, s, f, lv0, nfr);
-      e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    } else if (small_max > 0) {
-      switch (front_form(small_max)) {
-        case 1: e = launch_level<16, 64>(f, lv0, nfr, s); break;
-        case 2: e = launch_level<16, 256>(f, lv0, nfr, s); break;
-        case 3: e = launch_level<16, 1024>(f, lv0, nfr, s); break;
-        case 4: e = launch_level<8, 1934>(f, lv0, nfr, s); break;
-        default: e = launch_level<4, kFrontMaxM>(f, lv0, nfr, s); break;
+    if (one_max > 0) {
+      const int nfr = lv1 - big0;
+      switch (front_form(one_max)) {
+        case 2: e = launch_level<16, 256>(f, big0, nfr, s); break;
+        case 3: e = launch_level<16, 1024>(f, big0, nfr, s); break;
+        case 4: e = launch_level<8, 1934>(f, big0, nfr, s); break;
+        default: e = launch_level<4, kFrontMaxM>(f, big0, nfr, s); break;
       }
       if (e != hipSuccess) return e;
     }
     // the level's larger fronts, at most kBigLaunch per launch (grid y / z)
-    if (any_big)
-      for (int lb = f.big_ptr_host[L]; lb < f.big_ptr_host[L + 1]; lb += kBigLaunch)
-        if ((e = launch_big_fronts(f, lb, std::min(kBigLaunch, f.big_ptr_host[L + 1] - lb), s)) !=
-            hipSuccess)
-          return e;
+    for (int lb = f.big_ptr_host[L]; lb < f.big_ptr_host[L + 1]; lb += kBigLaunch)
+      if ((e = launch_big_fronts(f, lb, std::min(kBigLaunch, f.big_ptr_host[L + 1] - lb), s)) !=
+          hipSuccess)
+        return e;
   }
   // the backward solve's LDS holds a front's rows: the level's largest front
   // picks the instance (the largest fronts with 512 threads)
   for (int L = f.n_levels - 1; L >= 0; --L) {
-    const int lv0 = f.lv_ptr_host[L], nfr = f.lv_ptr_host[L + 1] - lv0;
+    const int32_t *cp = f.cls_host + 3 * L;
     const int mm = f.lv_maxm_host[L];
-    if (mm <= 64)
-      hipLaunchKernelGGL((front_bwd_kernel<64, kFB>), dim3(nfr), dim3(kFB), 0, s, f, lv0);
-    else if (mm <= 512)
-      hipLaunchKernelGGL((front_bwd_kernel<512, kFB>), dim3(nfr), dim3(kFB), 0, s, f, lv0);
-    else
-      hipLaunchKernelGGL((front_bwd_kernel<kFrontMaxM, kSolveBlock>), dim3(nfr),
-                         dim3(kSolveBlock), 0, s, f, lv0);
+    const int wave0 = cp[2] - cp[0] <= kWaveFronts ? cp[0] : cp[1];
+    if (wave0 > cp[0])
+      hipLaunchKernelGGL(front_tiny_bwd_kernel, dim3((wave0 - cp[0] + 63) / 64), dim3(64), 0, s,
+                         f, cp[0], wave0 - cp[0]);
+    if (cp[2] > wave0)
+      hipLaunchKernelGGL((front_bwd_kernel<64, kFB>), dim3(cp[2] - wave0), dim3(kFB), 0, s, f,
+                         wave0);
+    if (cp[3] > cp[2]) {
+      if (mm <= 512)
+        hipLaunchKernelGGL((front_bwd_kernel<512, kFB>), dim3(cp[3] - cp[2]), dim3(kFB), 0, s, f,
+                           cp[2]);
+      else
+        hipLaunchKernelGGL((front_bwd_kernel<kFrontMaxM, kSolveBlock>), dim3(cp[3] - cp[2]),
+                           dim3(kSolveBlock), 0, s, f, cp[2]);
+    }
   }
   hipLaunchKernelGGL(front_finish_kernel, dim3(f.n_comp), dim3(kFinishBlock), 0, s, f, a);
   if (f.n_fin_chunks > 0) {

@@ -280,6 +280,7 @@ struct SparseLuArgs {
 constexpr int kFrontMaxM = 3481;  // largest front a workgroup's panel holds
 // Fronts of more rows are factored by many workgroups per panel.
 constexpr int32_t kFrontBigM = 64;
+constexpr int kTinyM = 8;                // rows of a front factored by one thread
 constexpr int kBigW = 32;               // most columns of their panels
 constexpr int kMoveInts = 1 + 2 * kBigW;  // FrontArgs::mv per front
 constexpr int kBigLaunch = 65535;       // most large fronts per launch (grid y / z)
@@ -304,10 +305,12 @@ struct FrontArgs {
   double *lbuf = nullptr;
   const int32_t *active;
   const int32_t *gate = nullptr;  // stop word (LoadPtrs::gate)
-  const int32_t *lv_ptr_host, *lv_maxm_host;  // host arrays: the launch loop
+  // host arrays: the launch loop.  `lv` (and lv_host) list each level's
+  // fronts by size class, cls_host[3 L .. 3 L + 3] the classes' bounds
+  const int32_t *lv_maxm_host, *cls_host;
   // host copies for the many-workgroup form of fronts of more than big_m
   // rows
-  const int32_t *lv_host, *m_host, *k_host, *ch_ptr_host, *ch_host;
+  const int32_t *lv_host, *m_host;
   int32_t big_m = kFrontBigM;
   // those fronts grouped by level (device), with the host's level offsets
   const BigFront *big = nullptr, *big_host = nullptr;
