@@ -383,32 +383,108 @@ struct CompLu {
   std::vector<int32_t> lv_end, lv_mid, lv_long;  // per level, task indices
 };
 
-// Supernodal multifrontal plan from the elimination tree `parent` and the
-// strictly-lower column structures `ucol` (ascending) of a component in
-// pivot positions.  Supernodes: column j joins j - 1 when j is the parent
-// of j - 1 and L(:, j-1) = {j} + L(:, j) (other children of j then hang off
-// the supernode: their contribution rows lie in its rows).  Front s covers
-// columns [f, l) with rows R = [f, l) + L(:, l-1) (ascending); its dense
-// m x m block (row-major) receives the matrix entries whose smaller
-// position falls in [f, l), and the contribution blocks of its children.
-// Entry e is (ei[e], ej[e]) in positions.
-bool build_fronts(int32_t n, const std::vector<int32_t> &parent,
-                  const std::vector<std::vector<int32_t>> &ucol,
+// Fronts from the elimination tree `parent` and the strictly-lower column
+// structures `ucol` of a component: front_tree[s] lists front s's columns
+// (ascending, old positions; the last one's structure is the front's rows
+// below), children before parents and every front's columns last among its
+// subtree's, so that numbering them in this order is an equivalent
+// elimination order.
+//
+// The tree's height is what a factorisation waits for: a level costs a few
+// dependent launches (~15 us for fronts of a wavefront, ~40 us for large
+// ones), a column step of a front ~1 us.  So the deepest children of a front
+// join it together (a part of them would leave the height as it is) while the
+// columns that this makes serial -- all but the longest child's -- cost less
+// than the level: kMergeSmall of them up to kMergeRows rows, kMergeBig above,
+// where the zeros stored may cost kMergeFlops (~10 us).  A front does not
+// outgrow a wavefront this way, except with a child that adds no zeros.  5,000-gate logic: 18,215 fronts in 26 levels
+// before.
+constexpr int64_t kMergeRows = 64, kMergeSmall = 8, kMergeBig = 24, kMergeFlops = 30000000;
+
+std::vector<std::vector<int32_t>> front_tree(int32_t n, const std::vector<int32_t> &parent,
+                                             const std::vector<std::vector<int32_t>> &ucol) {
+  // flops of k pivots of an m-row front
+  auto cost = [](int64_t m, int64_t k) {
+    auto sq = [](int64_t x) { return (double)x * (double)(x + 1) * (double)(2 * x + 1) / 3.0; };
+    return sq(m - 1) - sq(m - 1 - k);
+  };
+  std::vector<std::vector<int32_t>> cols(n), kids(n);  // by a front's last column
+  std::vector<int32_t> height(n, 0);
+  for (int32_t j = 0; j < n; ++j) {
+    cols[j].push_back(j);
+    int64_t m = 1 + (int64_t)ucol[j].size(), k = 1;
+    while (!kids[j].empty()) {
+      int32_t top = 0;
+      for (int32_t c : kids[j]) top = std::max(top, height[c]);
+      int64_t sum = 0, most = 0, n_top = 0;
+      double parts = cost(m, k);
+      bool same = false;  // a child with this front's rows: no zeros
+      for (int32_t c : kids[j])
+        if (height[c] == top) {
+          const int64_t kc = (int64_t)cols[c].size();
+          same = n_top++ == 0 && (int64_t)ucol[c].size() == m;
+          sum += kc;
+          most = std::max(most, kc);
+          parts += cost(kc + (int64_t)ucol[c].size(), kc);
+        }
+      const bool small = m + sum <= kMergeRows;
+      if (m + sum > kFrontMaxM) break;
+      if (!same && ((m <= kMergeRows && !small) ||
+                    sum - most > (small ? kMergeSmall : kMergeBig) ||
+                    (!small && cost(m + sum, k + sum) - parts > (double)kMergeFlops)))
+        break;
+      std::vector<int32_t> left;
+      for (int32_t c : kids[j])
+        if (height[c] == top) {
+          cols[j].insert(cols[j].end(), cols[c].begin(), cols[c].end());
+          cols[c].clear();
+          left.insert(left.end(), kids[c].begin(), kids[c].end());
+          kids[c].clear();
+        } else {
+          left.push_back(c);
+        }
+      kids[j].swap(left);
+      m += sum;
+      k += sum;
+    }
+    for (int32_t c : kids[j]) height[j] = std::max(height[j], height[c] + 1);
+    std::sort(cols[j].begin(), cols[j].end());
+    if (parent[j] >= 0) kids[parent[j]].push_back(j);
+  }
+  // postorder (iterative: chains are as deep as the component is large)
+  std::vector<std::vector<int32_t>> out;
+  std::vector<std::pair<int32_t, size_t>> stack;
+  for (int32_t r = 0; r < n; ++r) {
+    if (parent[r] >= 0) continue;
+    stack.emplace_back(r, 0);
+    while (!stack.empty()) {
+      auto &top = stack.back();
+      if (top.second < kids[top.first].size()) {
+        const int32_t c = kids[top.first][top.second++];
+        stack.emplace_back(c, 0);
+      } else {
+        out.push_back(std::move(cols[top.first]));
+        stack.pop_back();
+      }
+    }
+  }
+  return out;
+}
+
+// Multifrontal plan of a component whose fronts own the positions
+// [first[s], first[s + 1]): front s covers these columns with rows R =
+// its columns + below[s] (ascending); its dense m x m block (row-major)
+// receives the matrix entries whose smaller position falls in its columns,
+// and the contribution blocks of its children.  Entry e is (ei[e], ej[e])
+// in positions.
+bool build_fronts(const std::vector<int32_t> &first,
+                  const std::vector<std::vector<int32_t>> &below,
                   const std::vector<int32_t> &ei, const std::vector<int32_t> &ej,
                   FrontLocal &F, std::string &err) {
-  std::vector<int32_t> nchild(n, 0);
-  for (int32_t j = 0; j < n; ++j)
-    if (parent[j] >= 0) nchild[parent[j]]++;
-  std::vector<int32_t> first;  // supernode starts
-  std::vector<int32_t> sn_of(n);
-  for (int32_t j = 0; j < n; ++j) {
-    const bool join = j > 0 && parent[j - 1] == j &&
-                      ucol[j - 1].size() == ucol[j].size() + 1;
-    if (!join) first.push_back(j);
-    sn_of[j] = (int32_t)first.size() - 1;
-  }
-  const int32_t ns = (int32_t)first.size();
-  first.push_back(n);
+  const int32_t ns = (int32_t)first.size() - 1;
+  std::vector<int32_t> sn_of(first[ns]);
+  for (int32_t s = 0; s < ns; ++s)
+    for (int32_t j = first[s]; j < first[s + 1]; ++j) sn_of[j] = s;
   F.m.resize(ns);
   F.k.resize(ns);
   F.height.assign(ns, 0);
@@ -416,14 +492,13 @@ bool build_fronts(int32_t n, const std::vector<int32_t> &parent,
   F.ro.assign(ns + 1, 0);
   std::vector<int32_t> spar(ns, -1);
   for (int32_t s = 0; s < ns; ++s) {
-    const int32_t f = first[s], l = first[s + 1];
-    const int32_t k = l - f, m = k + (int32_t)ucol[l - 1].size();
+    const int32_t k = first[s + 1] - first[s], m = k + (int32_t)below[s].size();
     F.k[s] = k;
     F.m[s] = m;
     F.max_m = std::max(F.max_m, m);
     F.fo[s + 1] = F.fo[s] + (int64_t)m * m;
     F.ro[s + 1] = F.ro[s] + m;
-    if (parent[l - 1] >= 0) spar[s] = sn_of[parent[l - 1]];
+    if (!below[s].empty()) spar[s] = sn_of[below[s][0]];
     // flops of the partial factorisation: per pivot a column scaling and a
     // rank-1 update of the trailing block
     for (int64_t j = 0; j < k; ++j) F.flops += (m - j - 1) + 2 * (m - j - 1) * (m - j - 1);
@@ -432,9 +507,8 @@ bool build_fronts(int32_t n, const std::vector<int32_t> &parent,
   F.cbmap.assign(F.ro[ns], -1);
   for (int32_t s = 0; s < ns; ++s) {
     int32_t *r = F.rows.data() + F.ro[s];
-    const int32_t f = first[s], l = first[s + 1];
-    for (int32_t j = f; j < l; ++j) *r++ = j;
-    for (int32_t i : ucol[l - 1]) *r++ = i;
+    for (int32_t j = first[s]; j < first[s + 1]; ++j) *r++ = j;
+    for (int32_t i : below[s]) *r++ = i;
   }
   auto local = [&](int32_t s, int32_t pos) -> int32_t {
     const int32_t *b = F.rows.data() + F.ro[s], *e = b + F.m[s];
@@ -642,7 +716,27 @@ void analyse_component_uncached(const Plan &plan, LuPlan &L, int32_t c,
     int64_t work = 0;  // multiply-adds: sum over pivots of (column count)^2
     for (int32_t k = 0; k < n; ++k) work += (int64_t)ucol[k].size() * (int64_t)ucol[k].size();
     if (fill > kLuMaxFill || work > kLuMaxOps || fronts_for(fill)) {
-      // too large for one workgroup's task lists: dense fronts
+      // too large for one workgroup's task lists: dense fronts, the
+      // component's positions renumbered by their tree
+      const std::vector<std::vector<int32_t>> tree = front_tree(n, parent, ucol);
+      std::vector<int32_t> first(1, 0), at(n), old(order);
+      for (const auto &cols : tree) {
+        int32_t q = first.back();
+        for (int32_t j : cols) at[j] = q++;
+        first.push_back(q);
+      }
+      std::vector<std::vector<int32_t>> below(tree.size());
+      for (size_t s = 0; s < tree.size(); ++s) {
+        for (int32_t i : ucol[tree[s].back()]) below[s].push_back(at[i]);
+        std::sort(below[s].begin(), below[s].end());
+      }
+      for (int32_t i = 0; i < n; ++i) order[at[i]] = old[i];
+      for (int32_t i = 0; i < n; ++i) {
+        pinv[order[i]] = i;
+        L.qcol[beg + i] = nodes[order[i]];
+        L.qpos[nodes[order[i]]] = i;
+        L.prow[beg + i] = nodes[row_of_col[order[i]]];
+      }
       std::vector<int32_t> rpos(n);
       for (int32_t i = 0; i < n; ++i) rpos[row_of_col[order[i]]] = i;
       std::vector<int32_t> ei, ej;
@@ -656,7 +750,7 @@ void analyse_component_uncached(const Plan &plan, LuPlan &L, int32_t c,
           ej.push_back(pinv[loc(col)]);
         }
       }
-      if (!build_fronts(n, parent, ucol, ei, ej, out.fr, out.err)) {
+      if (!build_fronts(first, below, ei, ej, out.fr, out.err)) {
         out.rc = XG_E_ARG;
         return;
       }
