@@ -412,9 +412,9 @@ int xg_lu_cache_set_limit(int64_t bytes);
 
 /* Fronts of more than big_m rows (default 64) are factored panel by panel
    across many workgroups (one workgroup per panel, then every column's row
-   swaps and U12 rows, then the trailing update in 64 x 64 tiles); smaller
-   ones by one workgroup each.  Both forms give the same bits.  No
-   counterpart in the reference (tuning and tests). */
+   swaps and U12 rows and the rows below, then the trailing update in 64 x 64
+   tiles); smaller ones by one wavefront or workgroup each.  All forms give
+   the same bits.  No counterpart in the reference (tuning and tests). */
 int xg_lu_front_set_big(xg_handle *h, int32_t big_m);
 
 /* Components too large for the task lists of xg_lu_info (more than 4 M

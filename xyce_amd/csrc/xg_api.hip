@@ -949,6 +949,27 @@ static bool upload_handle(xg_handle *H) {
       chk(o = h.upload(L.ops));
       u.ops = (const int2 *)o;
     }
+    {
+      // the packed lists of the components in LDS
+      std::vector<uint32_t> pt(2 * L.t_dst.size(), 0), po(L.ops.size() / 2, 0);
+      for (int32_t c = 0; c < u.n_comp; ++c) {
+        if (!L.in_lds[c] || !L.ok[c]) continue;
+        const int32_t t0 = L.lv_ptr[L.lv_comp[3 * (size_t)c]],
+                      t1 = L.lv_ptr[L.lv_comp[3 * (size_t)c + 3]];
+        const int32_t ob = t0 < t1 ? L.t_op[t0] : 0;
+        for (int32_t k = t0; k < t1; ++k) {
+          pt[2 * (size_t)k] = (uint32_t)L.t_dst[k] | (uint32_t)L.t_div[k] << 16;
+          pt[2 * (size_t)k + 1] =
+              (uint32_t)(L.t_op[k] - ob) | (uint32_t)(L.t_op[k + 1] - L.t_op[k]) << 16;
+          for (int32_t o = L.t_op[k]; o < L.t_op[k + 1]; ++o)
+            po[o] = (uint32_t)L.ops[2 * (size_t)o] | (uint32_t)L.ops[2 * (size_t)o + 1] << 16;
+        }
+      }
+      uint32_t *o;
+      chk(o = h.upload(pt));
+      u.ptasks = (const uint2 *)o;
+      chk(u.pops = h.upload(po));
+    }
     chk(u.ent_off = h.upload(L.ent_off));
     chk(u.ent_k = h.upload(L.ent_k));
     chk(u.ent_pos = h.upload(L.ent_pos));
@@ -967,14 +988,15 @@ static bool upload_handle(xg_handle *H) {
     f.n_fronts = (int32_t)L.fr_m.size();
     f.n_comp = u.n_comp;
     if (f.n_fronts > 0) {
-      // each level's fronts by size class
+      // each level's fronts by size class, those up to 64 rows by size
       h.fr_lv = L.fr_lv;
       h.fr_cls.assign(1, 0);
       for (size_t l = 0; l + 1 < L.fr_lv_ptr.size(); ++l) {
         const auto b = h.fr_lv.begin() + L.fr_lv_ptr[l], e = h.fr_lv.begin() + L.fr_lv_ptr[l + 1];
-        const auto t = std::stable_partition(
-            b, e, [&](int32_t s) { return L.fr_m[s] <= xg::kTinyM; });
-        const auto g = std::stable_partition(t, e, [&](int32_t s) { return L.fr_m[s] <= 64; });
+        const auto g = std::stable_partition(b, e, [&](int32_t s) { return L.fr_m[s] <= 64; });
+        std::stable_sort(b, g, [&](int32_t x, int32_t y) { return L.fr_m[x] < L.fr_m[y]; });
+        const auto t =
+            std::find_if(b, g, [&](int32_t s) { return L.fr_m[s] > xg::kTinyM; });
         h.fr_cls.push_back((int32_t)(t - h.fr_lv.begin()));
         h.fr_cls.push_back((int32_t)(g - h.fr_lv.begin()));
         h.fr_cls.push_back((int32_t)(e - h.fr_lv.begin()));
@@ -1095,6 +1117,31 @@ static bool upload_handle(xg_handle *H) {
         }
       }
       u.front = f.front_comp;
+    }
+    {
+      std::vector<xg::LuComp> lc((size_t)(u.n_comp > 0 ? u.n_comp : 0));
+      for (int32_t c = 0; c < u.n_comp; ++c) {
+        xg::LuComp &q = lc[c];
+        const int32_t *lv = L.lv_comp.data() + 3 * (size_t)c;
+        q.beg = P.comp_start[c];
+        q.n = P.comp_start[c + 1] - q.beg;
+        q.in_lds = L.in_lds[c] != 0;
+        q.ok = L.ok[c] != 0;
+        q.front = f.n_fronts > 0 && L.front_comp[c] != 0;
+        q.L0 = lv[0];
+        q.f1 = lv[1] - lv[0];
+        q.s1 = lv[2] - lv[0];
+        q.nlev = lv[3] - lv[0];
+        q.tbase = L.lv_ptr[lv[0]];
+        q.ntask = L.lv_ptr[lv[3]] - q.tbase;
+        q.obase = q.ntask ? L.t_op[q.tbase] : 0;
+        q.nops = q.ntask ? L.t_op[q.tbase + q.ntask] - q.obase : 0;
+        q.eb = L.ent_off[c];
+        q.ne = L.ent_off[c + 1] - q.eb;
+        q.voff = L.voff[c];
+        q.nv = (int32_t)(L.voff[c + 1] - L.voff[c]);
+      }
+      chk(u.comp = h.upload(lc));
     }
     if (ok && hipMemset(u.fallback, 0, sizeof(int32_t) * (u.n_comp > 0 ? u.n_comp : 1)) !=
                   hipSuccess)

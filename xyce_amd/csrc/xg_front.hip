@@ -33,6 +33,7 @@
 #include <cfloat>
 
 #include "xg_internal.h"
+#include "xg_lu_dev.h"
 
 namespace xg {
 
@@ -83,26 +84,6 @@ __device__ __forceinline__ double blk_reduce(double v, double *sv, bool is_max) 
   const double r = sv[0];
   __syncthreads();
   return r;
-}
-
-// Division by a pivot shared by many rows: the pivot's mantissa p, its
-// reciprocal r and minus its exponent, then per row a quotient and one
-// correction with the exact remainder (four operations instead of the ~11 of
-// a full division; the last bit's error is that of one rounding but for
-// rare double roundings).  Scaling by the exponent keeps the whole range.
-// Every form below divides this way, so all give the same bits.
-struct Pivot {
-  double p, r;
-  int e;
-};
-__device__ __forceinline__ Pivot make_pivot(double v) {
-  const double p = __builtin_amdgcn_frexp_mant(v);
-  return {p, 1.0 / p, -__builtin_amdgcn_frexp_exp(v)};
-}
-__device__ __forceinline__ double divide(double a, const Pivot &v) {
-  const double x = __builtin_amdgcn_ldexp(a, v.e);
-  const double q = x * v.r;
-  return fma(fma(-q, v.p, x), v.r, q);
 }
 
 // Partial LU of the m x m row-major front A and its right-hand side w (the
@@ -250,14 +231,6 @@ __device__ bool front_factor(double *A, double *w, int m, int k, double *P, doub
 
 __device__ __forceinline__ bool front_skip(const FrontArgs &f, int c) {
   return (f.gate && *f.gate) || (f.active && !f.active[c]) || f.bad[c];
-}
-
-// p[i], or 0 where it may not be read (p[0] may): a select, no branch, so
-// that a run of these loads is in flight together (behind `cond ? p[i] : 0`
-// with a short-circuit the compiler waits for each one).
-__device__ __forceinline__ double load_if(bool ok, const double *p, int64_t i) {
-  const double v = p[ok ? i : 0];
-  return ok ? v : 0.0;
 }
 
 // Clears the fronts and the failure flags and sets the right-hand-side
@@ -431,10 +404,6 @@ __device__ __forceinline__ unsigned lanes_max(unsigned v) {
   if (kSteps > 5) v = dpp_max<0x143, 0xc>(v);
   return (unsigned)__builtin_amdgcn_readlane((int)v, (1 << kSteps) - 1);
 }
-__device__ __forceinline__ double read_lane(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
 // The lane (of the first 2^kSteps) with the largest v >= 0, the smallest p
 // on ties (lanes holding no candidate: v = 0, which never wins over one).
 // Magnitudes order as their bits do: the high words first, the low ones
@@ -487,7 +456,8 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 template <int NW, int kNT, int kCT>
 __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int lb, int kb) {
   constexpr int R = kNT / 4, W = 16 * kCT, kRows = 16 * kNT;
-  static_assert(kNT % 4 == 0 && (NW == 1 || NW == 4 || NW == 8), "rows per lane, search");
+  static_assert(kNT % 4 == 0 && NW <= 16 && (NW & (NW - 1)) == 0, "rows per lane, search");
+  constexpr int kSteps = NW >= 16 ? 4 : NW >= 8 ? 3 : NW >= 4 ? 2 : 1;
   __shared__ __align__(16) double S[NW][kRows][4];
   __shared__ __align__(16) double srow[2][4][NW][4];
   __shared__ double sval[2][4][NW], srcp[2][4][NW], raw[4][W];
@@ -590,7 +560,7 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
           // the best wavefront: lanes 0..NW-1 hold the candidates
           const double cv = lane < NW ? sval[par][j][lane] : 0.0;
           const int cp = lane < NW ? spos[par][j][lane] : 0x7fffffff;
-          bw = lane_of_max<NW == 8 ? 3 : 2>(cv, cp);
+          bw = lane_of_max<kSteps>(cv, cp);
           best = read_lane(cv, bw);
         }
         if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
@@ -1088,22 +1058,6 @@ __global__ void __launch_bounds__(kFB) front_update_kernel(FrontArgs f, int lb, 
   }
 }
 
-// Sum over the 16 lanes of a row, the same bits in every lane: neighbours,
-// then pairs, quads and halves (each step adds two mirror images).
-template <int kCtrl>
-__device__ __forceinline__ double dpp_add(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  return v + __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, kCtrl, 0xf, 0xf, false),
-                              __builtin_amdgcn_update_dpp(lo, lo, kCtrl, 0xf, 0xf, false));
-}
-__device__ __forceinline__ double sum8(double v) {
-  return dpp_add<0x141>(dpp_add<0x4e>(dpp_add<0xb1>(v)));
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v = dpp_add<0x140>(sum8(v));
-  return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
-}
-
 // Backward solve of one level's fronts (levels from the root down): the
 // rows below the fully summed block are solved already (by ancestors).
 // First the right-hand side less the solved rows below, a wavefront per
@@ -1544,16 +1498,26 @@ hipError_t launch_fronts(const FrontArgs &f, const SparseLuArgs &a, hipStream_t 
       hipLaunchKernelGGL(front_tiny_kernel, dim3((wave0 - lv0 + 63) / 64), dim3(64), 0, s, f,
                          lv0, wave0 - lv0);
     if (big0 > wave0) {
-      int32_t mx = 0;
-      for (int q = wave0; q < big0; ++q) mx = std::max(mx, f.m_host[f.lv_host[q]]);
+      // (they are in order of size: a level of many takes a launch per tile
+      // count, so that the small ones have the registers and LDS of theirs)
+      for (int q0 = wave0; q0 < big0;) {
+        int q1 = big0;
+        int32_t mx = f.m_host[f.lv_host[big0 - 1]];
+        if (big0 - wave0 > kWaveFronts) {
+          mx = std::min(64, f.m_host[f.lv_host[q0]] / 16 * 16 + 15);
+          q1 = q0 + 1;
+          while (q1 < big0 && f.m_host[f.lv_host[q1]] <= mx) ++q1;
+        }
 #define XG_WAVE(NT, CT) \
-  hipLaunchKernelGGL((front_wave_kernel<NT, CT>), dim3(big0 - wave0), dim3(64), 0, s, f, wave0)
-      if (mx <= 15) XG_WAVE(1, 1);
-      else if (mx <= 31) XG_WAVE(2, 2);
-      else if (mx <= 47) XG_WAVE(3, 3);
-      else if (mx <= 63) XG_WAVE(4, 4);
-      else XG_WAVE(4, 5);
+  hipLaunchKernelGGL((front_wave_kernel<NT, CT>), dim3(q1 - q0), dim3(64), 0, s, f, q0)
+        if (mx <= 15) XG_WAVE(1, 1);
+        else if (mx <= 31) XG_WAVE(2, 2);
+        else if (mx <= 47) XG_WAVE(3, 3);
+        else if (mx <= 63) XG_WAVE(4, 4);
+        else XG_WAVE(4, 5);
 #undef XG_WAVE
+        q0 = q1;
+      }
     }
     if (one_max > 0) {
       const int nfr = lv1 - big0;

@@ -246,6 +246,16 @@ struct DenseSolveArgs {
 // read L from the factors and y from the vector.
 constexpr int32_t kLuFwdTask = -3;
 
+// One component of the sparse LU as its workgroup reads it.
+struct LuComp {
+  int32_t beg, n;                  // positions
+  int32_t in_lds, ok, front;       // SparseLuArgs::in_lds, ok, front
+  int32_t L0, f1, s1, nlev;        // first level; levels of the phases, from it
+  int32_t tbase, ntask, obase, nops;
+  int32_t eb, ne;                  // Jacobian entries
+  int32_t nv;                      // values, in LDS or at voff of val_work
+  int64_t voff;
+};
 // Static-pivot sparse LU per component (task lists of lu_analyse).
 struct SparseLuArgs {
   int32_t n_comp = 0;
@@ -259,6 +269,12 @@ struct SparseLuArgs {
   const int32_t *lv_comp, *lv_ptr, *lv_mid, *lv_long;
   const int4 *tasks;              // {dst, div, first op, end op}
   const int2 *ops;
+  // the lists of components in LDS, packed: destination, divisor
+  // (signed), first op (of the component's) and number of ops, 16 bits each;
+  // an op's two positions, 16 bits each
+  const LuComp *comp = nullptr;
+  const uint2 *ptasks = nullptr;
+  const uint32_t *pops = nullptr;
   const int32_t *ent_off, *ent_k, *ent_pos, *ent_col, *ent_rs;
   double *Jp, *bp;                // J in entry order, rhs in position order
   int32_t n_ent = 0, n_nodes = 0;

@@ -20,8 +20,10 @@
 // component that fails is flagged, its iterate left as it was, and the
 // dense partial-pivoting kernel launched right after refactors just those.
 #include <cfloat>
+#include <type_traits>
 
 #include "xg_internal.h"
+#include "xg_lu_dev.h"
 
 namespace xg {
 
@@ -29,6 +31,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kLdsBytes = 144 * 1024;  // factors, vector and task lists
+static_assert(kLdsBytes / 8 < 32768, "packed task lists hold 15-bit numbers");
 
 __device__ __forceinline__ double blk_max(double v, double *sv) {
   const int t = threadIdx.x;
@@ -58,94 +61,207 @@ __device__ __forceinline__ double blk_sum(double v, double *sv) {
 
 __host__ __device__ constexpr int64_t align16(int64_t b) { return (b + 15) & ~(int64_t)15; }
 
-// The task lists of one component, with op ranges relative to `ops` and
-// level pointers relative to `tasks`.
-struct Lists {
-  const int4 *tasks;
-  const int2 *ops;
-  const int32_t *lvp, *lvm, *lvl;  // level -> first task, first mid, first long
-  int obase;  // subtracted from the ops fields of tasks (0 once staged)
+// A task as the levels run it: destination, divisor, first op and number of
+// ops; an op's two operand positions.
+struct Task {
+  int dst, div, o0, m;
 };
 
-// Finishes a task value: division by the pivot (factor and backward
-// solve) and the factor's acceptance checks.
+// The task lists of one component, level pointers relative to `tasks`.  In
+// LDS (kLds) tasks and ops are packed into 8 and 4 bytes (SparseLuArgs::
+// ptasks, pops): half the bytes to stage on every solve and one LDS word per
+// op.  Every number of a component that fits in LDS fits in 15 bits (144 KB
+// hold at most 18,432 values or ops).
+template <bool kLds>
+struct Lists {
+  using RawTask = std::conditional_t<kLds, uint2, int4>;
+  using RawOp = std::conditional_t<kLds, uint32_t, int2>;
+  const RawTask *tasks;
+  const RawOp *ops;
+  const int32_t *lvp, *lvm, *lvl;  // level -> first task, first mid, first long
+  static __device__ __forceinline__ Task task(const RawTask &v) {
+    if constexpr (kLds)
+      return {(int)(v.x & 0xffff), (int)v.x >> 16, (int)(v.y & 0xffff), (int)(v.y >> 16)};
+    else
+      return {v.x, v.y, v.z, v.w - v.z};
+  }
+  // op j of a task, past its end one of its own (whose operands may be read,
+  // too), of a task without ops the positions 0
+  __device__ __forceinline__ RawOp op_of(const Task &t, int j) const {
+    const RawOp v = ops[t.m > 0 ? t.o0 + min(j, t.m - 1) : 0];
+    if constexpr (kLds)
+      return t.m > 0 ? v : 0;
+    else
+      return t.m > 0 ? v : RawOp{0, 0};
+  }
+  static __device__ __forceinline__ int2 op(const RawOp &v) {
+    if constexpr (kLds)
+      return {(int)(v & 0xffff), (int)(v >> 16)};
+    else
+      return v;
+  }
+};
+
+// Finishes a task value: division by the pivot d (factor and backward
+// solve; read with the task's operands) and the factor's acceptance checks.
 template <int kPhase>
-__device__ __forceinline__ void finish_task(const int4 &tk, double s, double *val,
+__device__ __forceinline__ void finish_task(const Task &tk, double s, double d, double *val,
                                             double *vec, int &bad) {
   if (kPhase == 0) {
-    if (tk.y == kLuFwdTask) {  // a forward-substitution row (y in vec)
-      vec[tk.x] = s;
+    if (tk.div == kLuFwdTask) {  // a forward-substitution row (y in vec)
+      vec[tk.dst] = s;
       return;
     }
-    if (tk.y >= 0) {
-      s = s / val[tk.y];
+    if (tk.div >= 0) {  // (every task of a level or none: skipped as a whole)
+      s = divide(s, make_pivot(d));
       bad |= !(fabs(s) <= DBL_MAX);  // infinite or NaN
-    } else if (tk.y == -2) {
+    } else if (tk.div == -2) {
       bad |= !(fabs(s) > 0.0) || isinf(s);
     }
-    val[tk.x] = s;
+    val[tk.dst] = s;
   } else {
-    vec[tk.x] = kPhase == 2 ? s / val[tk.y] : s;
+    vec[tk.dst] = kPhase == 2 ? divide(s, make_pivot(d)) : s;
   }
 }
 
-// One level.  Short tasks (at most four terms): one thread each, the terms'
-// operands loaded together, then summed in list order.  Mid tasks: eight
-// lanes each, long tasks (rows of supply rails, which touch most of the
-// circuit): a wavefront each; lane-strided partial sums folded by a fixed
-// butterfly.  The association is fixed by the plan, so results do not
-// depend on the launch.
-template <int kPhase>
-__device__ __forceinline__ void run_level(const Lists &ls, int L, double *val,
-                                          double *vec, int &bad) {
-  const int k0 = ls.lvp[L], km = ls.lvm[L], kl = ls.lvl[L], k1 = ls.lvp[L + 1];
+// The levels [L0, L1).  Short tasks (at most four terms): one thread each,
+// the terms' operands loaded together, then summed in list order.  Mid
+// tasks: eight lanes each, long tasks (rows of supply rails, which touch
+// most of the circuit): a wavefront each; lane-strided partial sums folded
+// by a fixed tree.  The association is fixed by the plan, so results do
+// not depend on the launch.
+//
+// A level is one dependent step and its length is its latency, so it waits
+// for one LDS round trip, the operands': the level bounds are in lanes of
+// registers, a thread's first short and first mid task are read two levels
+// ahead and their ops one level ahead, kept as read until they are used.
+// (Bounds, task, ops and operands in turn were 1700 cycles a level.)  Mid
+// tasks start from the last wavefront and long ones from the second, so
+// that in a level of few tasks they run beside the short ones.
+template <int kPhase, bool kLds>
+__device__ __forceinline__ void run_levels(const Lists<kLds> &ls, int L0, int L1, double *val,
+                                           double *vec, int &bad) {
+  using RawTask = typename Lists<kLds>::RawTask;
+  using RawOp = typename Lists<kLds>::RawOp;
+  if (L0 >= L1) return;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int mid = (kBlock - 1 - t) >> 3, sub = t & 7;
+  const int lng = (wave + kBlock / 64 - 1) % (kBlock / 64);
   const double *src0 = kPhase == 0 ? val : vec;
-  for (int k = k0 + (int)threadIdx.x; k < km; k += kBlock) {
-    const int4 tk = ls.tasks[k];
-    const double *src = kPhase == 0 && tk.y == kLuFwdTask ? vec : src0;
-    const int o0 = tk.z - ls.obase, m = tk.w - tk.z;
+  // lane i: the bounds of level base + i
+  int base = 0, bp = 0, bm = 0, bl = 0;
+  auto fill = [&](int L) {
+    base = L;
+    bp = ls.lvp[min(L + lane, L1)];
+    bm = ls.lvm[min(L + lane, L1 - 1)];
+    bl = ls.lvl[min(L + lane, L1 - 1)];
+  };
+  struct Ahead {  // a thread's first short and mid task of a level
+    RawTask st, mt;
+    bool s_on, m_on;
+  };
+  auto tasks_of = [&](int L) {
+    const int i = min(L, L1 - 1) - base;
+    const int k0 = __builtin_amdgcn_readlane(bp, i), km = __builtin_amdgcn_readlane(bm, i),
+              kl = __builtin_amdgcn_readlane(bl, i);
+    Ahead a;
+    a.s_on = k0 + t < km;
+    a.m_on = km + mid < kl;
+    a.st = ls.tasks[a.s_on ? k0 + t : k0];
+    a.mt = ls.tasks[a.m_on ? km + mid : k0];
+    return a;
+  };
+  struct Ops {
+    RawOp s[4], m[2];
+  };
+  auto ops_of = [&](const Ahead &a) {
+    const Task st = ls.task(a.st), mt = ls.task(a.mt);
+    Ops q;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q.s[j] = ls.op_of(st, j);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) q.m[j] = ls.op_of(mt, sub + 8 * j);
+    return q;
+  };
+  auto short_task = [&](const Task &tk, const RawOp *raw, bool on) {
+    const double *src = kPhase == 0 && tk.div == kLuFwdTask ? vec : src0;
     double a[4], b[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (j < m) {
-        const int2 q = ls.ops[o0 + j];
-        a[j] = val[q.x];
-        b[j] = src[q.y];
-      }
+      const int2 q = ls.op(raw[j]);
+      a[j] = val[q.x];
+      b[j] = src[q.y];
     }
-    double s = src[tk.x];
+    double s = src[tk.dst];
+    const double d = val[max(tk.div, 0)];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j < m) s = s - a[j] * b[j];
-    finish_task<kPhase>(tk, s, val, vec, bad);
-  }
-  {
-    const int grp = threadIdx.x >> 3, sub = threadIdx.x & 7;
-    for (int k = km + grp; k < kl; k += kBlock / 8) {
-      const int4 tk = ls.tasks[k];
-      const double *src = kPhase == 0 && tk.y == kLuFwdTask ? vec : src0;
-      const int o0 = tk.z - ls.obase, o1 = tk.w - ls.obase;
+    for (int j = 0; j < 4; ++j) {
+      const double n = s - a[j] * b[j];
+      s = j < tk.m ? n : s;
+    }
+    if (on) finish_task<kPhase>(tk, s, d, val, vec, bad);
+  };
+  auto mid_task = [&](const Task &tk, const RawOp *raw) {
+    const double *src = kPhase == 0 && tk.div == kLuFwdTask ? vec : src0;
+    const double d = val[max(tk.div, 0)], s0 = src[tk.dst];
+    double p = 0.0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const bool in = sub + 8 * j < tk.m;
+      const int2 q = ls.op(raw[j]);
+      const double n = p + val[q.x] * src[q.y];
+      p = in ? n : p;
+    }
+    for (int o = sub + 16; o < tk.m; o += 8) {
+      const int2 r = ls.op(ls.ops[tk.o0 + o]);
+      p = p + val[r.x] * src[r.y];
+    }
+    p = sum8(p);
+    if (sub == 0) finish_task<kPhase>(tk, s0 - p, d, val, vec, bad);
+  };
+  fill(L0);
+  Ahead a0 = tasks_of(L0), a1 = tasks_of(L0 + 1);
+  Ops q0 = ops_of(a0);
+  for (int L = L0; L < L1; ++L) {
+    if (L - base > 60) fill(L);
+    const int i = L - base;
+    const int k0 = __builtin_amdgcn_readlane(bp, i), km = __builtin_amdgcn_readlane(bm, i),
+              kl = __builtin_amdgcn_readlane(bl, i), k1 = __builtin_amdgcn_readlane(bp, i + 1);
+    const Ops q1 = ops_of(a1);
+    const Ahead a2 = tasks_of(L + 2);
+    if (k0 + (t & ~63) < km) short_task(ls.task(a0.st), q0.s, a0.s_on);
+    for (int k = k0 + t + kBlock; k < km; k += kBlock) {
+      const Task tk = ls.task(ls.tasks[k]);
+      RawOp q[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[j] = ls.op_of(tk, j);
+      short_task(tk, q, true);
+    }
+    if (a0.m_on) mid_task(ls.task(a0.mt), q0.m);
+    for (int k = km + mid + kBlock / 8; k < kl; k += kBlock / 8) {
+      const Task tk = ls.task(ls.tasks[k]);
+      RawOp q[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[j] = ls.op_of(tk, sub + 8 * j);
+      mid_task(tk, q);
+    }
+    for (int k = kl + lng; k < k1; k += kBlock / 64) {
+      const Task tk = ls.task(ls.tasks[k]);
+      const double *src = kPhase == 0 && tk.div == kLuFwdTask ? vec : src0;
+      const double d = val[max(tk.div, 0)], s0 = src[tk.dst];
       double p = 0.0;
-      for (int o = o0 + sub; o < o1; o += 8) {
-        const int2 q = ls.ops[o];
+#pragma unroll 4
+      for (int o = lane; o < tk.m; o += 64) {
+        const int2 q = ls.op(ls.ops[tk.o0 + o]);
         p = p + val[q.x] * src[q.y];
       }
-      for (int off = 4; off >= 1; off >>= 1) p = p + __shfl_xor(p, off);
-      if (sub == 0) finish_task<kPhase>(tk, src[tk.x] - p, val, vec, bad);
+      p = wave_sum(p);
+      if (lane == 0) finish_task<kPhase>(tk, s0 - p, d, val, vec, bad);
     }
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int k = kl + wave; k < k1; k += kBlock / 64) {
-    const int4 tk = ls.tasks[k];
-    const double *src = kPhase == 0 && tk.y == kLuFwdTask ? vec : src0;
-    const int o0 = tk.z - ls.obase, o1 = tk.w - ls.obase;
-    double p = 0.0;
-    for (int o = o0 + lane; o < o1; o += 64) {
-      const int2 q = ls.ops[o];
-      p = p + val[q.x] * src[q.y];
-    }
-    for (int off = 32; off >= 1; off >>= 1) p = p + __shfl_xor(p, off);
-    if (lane == 0) finish_task<kPhase>(tk, src[tk.x] - p, val, vec, bad);
+    __syncthreads();
+    a0 = a1;
+    a1 = a2;
+    q0 = q1;
   }
 }
 
@@ -168,12 +284,15 @@ __global__ void __launch_bounds__(kBlock) sparse_lu_kernel(SparseLuArgs a) {
   __shared__ double sv[kBlock];
   const int c = blockIdx.x;
   const int t = threadIdx.x;
+  // (the component in one load, beside the stop word and its activity)
+  const LuComp q = a.comp[c];
+  const bool off = a.active && !a.active[c];
   if (a.gate && *a.gate) return;
-  if ((a.in_lds[c] != 0) != kLds) return;  // the other form
-  const int beg = a.cstart[c], n = a.cstart[c + 1] - beg;
-  const int64_t nv = a.voff[c + 1] - a.voff[c];
+  if (q.in_lds != (kLds ? 1 : 0)) return;  // the other form
+  const int beg = q.beg, n = q.n;
+  const int64_t nv = q.nv;
   double *stats = a.stats + 4 * (size_t)c;
-  if (a.active && !a.active[c]) {
+  if (off) {
     if (t == 0) {
       stats[0] = 0.0;
       stats[1] = 0.0;
@@ -183,21 +302,18 @@ __global__ void __launch_bounds__(kBlock) sparse_lu_kernel(SparseLuArgs a) {
     }
     return;
   }
-  if (a.front && a.front[c]) {  // the dense-front kernels solve it
+  if (q.front) {  // the dense-front kernels solve it
     if (t == 0) a.fallback[c] = 0;
     return;
   }
-  if (!a.ok[c]) {  // structurally singular under matching: dense kernel
+  if (!q.ok) {  // structurally singular under matching: dense kernel
     if (t == 0) a.fallback[c] = 1;
     return;
   }
-  const int32_t *lv = a.lv_comp + 3 * (size_t)c;
-  const int L0 = lv[0], nlev = lv[3] - lv[0];
-  const int tbase = a.lv_ptr[L0], ntask = a.lv_ptr[lv[3]] - tbase;
-  const int obase = ntask ? a.tasks[tbase].z : 0;
-  const int nops = ntask ? a.tasks[tbase + ntask - 1].w - obase : 0;
+  const int L0 = q.L0, nlev = q.nlev, tbase = q.tbase, ntask = q.ntask, obase = q.obase,
+            nops = q.nops;
   double *val, *vec;
-  Lists ls;
+  Lists<kLds> ls{};
   if (kLds) {
     // stage: [values][vector][tasks][ops][level pointers]
     char *p = lds;
@@ -205,36 +321,46 @@ __global__ void __launch_bounds__(kBlock) sparse_lu_kernel(SparseLuArgs a) {
     p += align16(nv * 8);
     vec = (double *)p;
     p += align16((int64_t)n * 8);
-    int4 *tk = (int4 *)p;
-    p += (int64_t)ntask * 16;
-    int2 *op = (int2 *)p;
-    p += align16((int64_t)nops * 8);
+    uint2 *tk = (uint2 *)p;
+    p += align16((int64_t)ntask * 8);
+    uint32_t *op = (uint32_t *)p;
+    p += align16((int64_t)nops * 4);
     int32_t *lvp = (int32_t *)p;
     int32_t *lvm = lvp + nlev + 1;
     int32_t *lvl = lvm + nlev;
-    for (int k = t; k < ntask; k += kBlock) tk[k] = a.tasks[tbase + k];
-    for (int k = t; k < nops; k += kBlock) op[k] = a.ops[obase + k];
+#pragma unroll 8
+    for (int k = t; k < ntask; k += kBlock) tk[k] = a.ptasks[tbase + k];
+#pragma unroll 8
+    for (int k = t; k < nops; k += kBlock) op[k] = a.pops[obase + k];
     for (int k = t; k <= nlev; k += kBlock) lvp[k] = a.lv_ptr[L0 + k] - tbase;
     for (int k = t; k < nlev; k += kBlock) {
       lvm[k] = a.lv_mid[L0 + k] - tbase;
       lvl[k] = a.lv_long[L0 + k] - tbase;
     }
-    ls = Lists{tk, op, lvp, lvm, lvl, obase};
+    ls.tasks = (const typename Lists<kLds>::RawTask *)tk;
+    ls.ops = (const typename Lists<kLds>::RawOp *)op;
+    ls.lvp = lvp;
+    ls.lvm = lvm;
+    ls.lvl = lvl;
   } else {
-    val = a.val_work + a.voff[c];
+    val = a.val_work + q.voff;
     vec = a.vec_work + beg;
-    // global lists: level pointers stay absolute, ops absolute
-    ls = Lists{a.tasks, a.ops, a.lv_ptr + L0, a.lv_mid + L0, a.lv_long + L0, 0};
+    // global lists: level pointers and ops stay absolute
+    ls.tasks = (const typename Lists<kLds>::RawTask *)a.tasks;
+    ls.ops = (const typename Lists<kLds>::RawOp *)a.ops;
+    ls.lvp = a.lv_ptr + L0;
+    ls.lvm = a.lv_mid + L0;
+    ls.lvl = a.lv_long + L0;
   }
   const int32_t *qcol = a.qcol + beg;
   // the component's Jacobian entries and right-hand side, already laid out
   // contiguously by the permute kernel
-  const int eb = a.ent_off[c], ne = a.ent_off[c + 1] - eb;
+  const int eb = q.eb, ne = q.ne;
   const double *jp = a.Jp + eb, *bp = a.bp + beg;
   const int32_t *epos = a.ent_pos + eb, *ecol = a.ent_col + eb, *ers = a.ent_rs + beg + c;
   for (int64_t e = t; e < nv; e += kBlock) val[e] = 0.0;
   __syncthreads();
-#pragma unroll 4
+#pragma unroll 8
   for (int j = t; j < ne; j += kBlock) val[epos[j]] = jp[j];
   double rmax = 0.0;
   for (int i = t; i < n; i += kBlock) {
@@ -244,39 +370,54 @@ __global__ void __launch_bounds__(kBlock) sparse_lu_kernel(SparseLuArgs a) {
   }
   const double max_rhs = blk_max(rmax, sv);  // includes the barriers
   // ---- factor
-  const int f1 = lv[1] - L0, s1 = lv[2] - L0;
+  const int f1 = q.f1, s1 = q.s1;
   int bad = 0;
-  for (int L = 0; L < f1; ++L) {
-    run_level<0>(ls, L, val, vec, bad);
-    __syncthreads();
-  }
+  run_levels<0>(ls, 0, f1, val, vec, bad);
   if (__syncthreads_or(bad)) {
     if (t == 0) a.fallback[c] = 1;
     return;
   }
   // ---- L y = P b (unit diagonal), then U x' = y, in place
-  for (int L = f1; L < s1; ++L) {
-    run_level<1>(ls, L, val, vec, bad);
-    __syncthreads();
-  }
-  for (int L = s1; L < nlev; ++L) {
-    run_level<2>(ls, L, val, vec, bad);
-    __syncthreads();
-  }
+  run_levels<1>(ls, f1, s1, val, vec, bad);
+  run_levels<2>(ls, s1, nlev, val, vec, bad);
   // ---- backward error of the solution against the unfactored rows
+  // (rows of more than kWaveRow entries, the supply rails, by a wavefront
+  // each: in one thread a 600-entry row took 13 us of the 70)
+  constexpr int kWaveRow = 32;
   double rm = 0.0, am = 0.0, xm = 0.0;
-  for (int i = t; i < n; i += kBlock) {
-    double r = bp[i], as = 0.0;
-    const int j0 = ers[i], j1 = ers[i + 1];
-#pragma unroll 4
-    for (int j = j0; j < j1; ++j) {
-      const double v = jp[j];
-      r = r - v * vec[ecol[j]];
-      as = as + fabs(v);
+  for (int i0 = 0; i0 < n; i0 += kBlock) {
+    const int i = i0 + t;
+    const int j0 = i < n ? ers[i] : 0, j1 = i < n ? ers[i + 1] : 0;
+    const bool wide = j1 - j0 > kWaveRow;
+    if (i < n) xm = fmax(xm, fabs(vec[i]));
+    if (i < n && !wide) {
+      double r = bp[i], as = 0.0;
+#pragma unroll 8
+      for (int j = j0; j < j1; ++j) {
+        const double v = jp[j];
+        r = r - v * vec[ecol[j]];
+        as = as + fabs(v);
+      }
+      rm = fmax(rm, fabs(r));
+      am = fmax(am, as);
     }
-    rm = fmax(rm, fabs(r));
-    am = fmax(am, as);
-    xm = fmax(xm, fabs(vec[i]));
+    unsigned long long mask = __ballot(wide);
+    while (mask) {  // this wavefront's wide rows
+      const int l = __ffsll(mask) - 1;
+      mask &= mask - 1;
+      const int w0 = __builtin_amdgcn_readlane(j0, l), w1 = __builtin_amdgcn_readlane(j1, l);
+      double r = 0.0, as = 0.0;
+#pragma unroll 4
+      for (int j = w0 + (t & 63); j < w1; j += 64) {
+        const double v = jp[j];
+        r = r + v * vec[ecol[j]];
+        as = as + fabs(v);
+      }
+      r = wave_sum(r);
+      as = wave_sum(as);
+      rm = fmax(rm, fabs(bp[__builtin_amdgcn_readlane(i, l)] - r));
+      am = fmax(am, as);
+    }
   }
   rm = blk_max(rm, sv);
   am = blk_max(am, sv);
