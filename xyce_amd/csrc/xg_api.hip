@@ -1176,7 +1176,8 @@ static bool upload_handle(xg_handle *H) {
   auto up_prog = [&](const xg::ReduceProgram &rp, xg::ReduceDev &rd) {
     rd.n_short4 = (int32_t)rp.sdst4.size();
     rd.n_short = (int32_t)rp.sdst.size();
-    rd.n_chunk = (int32_t)rp.cdst.size();
+    rd.n_chunk = rp.n_chunk;
+    rd.n_wide = (int32_t)rp.wtgt.size();
     rd.n_multi = (int32_t)rp.mtgt.size();
     rd.n_zero = (int32_t)rp.zidx.size();
     rd.pbase = rp.pbase;
@@ -1190,6 +1191,8 @@ static bool upload_handle(xg_handle *H) {
     chk(rd.cdst = h.upload(rp.cdst));
     chk(rd.mtgt = h.upload(rp.mtgt));
     chk(rd.mchunk = h.upload(rp.mchunk));
+    chk(rd.wtgt = h.upload(rp.wtgt));
+    chk(rd.wchunk = h.upload(rp.wchunk));
   };
   chk(h.partial = h.alloc<double>((size_t)P.n_partials));
   for (int k = 0; k < 4; ++k) up_prog(P.red_vec[k], h.red_vec[k]);

@@ -67,7 +67,9 @@ enum Mos1Slot : int {
 //    chunks of at most kChunk.  Chunk c covers src[cptr[c] .. cptr[c+1]); if
 //    it is the whole segment of entry e then cdst[c] = e, else -1 and its
 //    sum goes to partial[pbase + c].  Multi-chunk entry i (mtgt[i]) owns
-//    chunks [mchunk[2i], mchunk[2i+1]);
+//    chunks [mchunk[2i], mchunk[2i+1]).  Entries of 2 to 64 chunks (wtgt[i],
+//    chunks [wchunk[2i], wchunk[2i+1]), after the first n_chunk) are folded
+//    by one wavefront, a lane per chunk, with no second pass;
 //  * zidx lists the entries no source reaches (and the ground slot, row and
 //    column), which the overwrite output mode sets to +0.0.
 constexpr int32_t kShort = 8;
@@ -79,7 +81,8 @@ struct ReduceProgram {
   std::vector<int32_t> ssrc, sdst;
   std::vector<int32_t> src;
   std::vector<int32_t> cptr, cdst;
-  std::vector<int32_t> mtgt, mchunk;
+  std::vector<int32_t> mtgt, mchunk, wtgt, wchunk;
+  int32_t n_chunk = 0;
   std::vector<int32_t> zidx;
   int32_t pbase = 0;
 };
@@ -90,6 +93,7 @@ struct ReduceDev {
   int32_t n_short = 0;
   int32_t n_chunk = 0;
   int32_t n_multi = 0;
+  int32_t n_wide = 0;
   int32_t n_zero = 0;
   int32_t pbase = 0;
   int32_t *ssrc4 = nullptr;
@@ -101,6 +105,8 @@ struct ReduceDev {
   int32_t *cdst = nullptr;
   int32_t *mtgt = nullptr;
   int32_t *mchunk = nullptr;
+  int32_t *wtgt = nullptr;
+  int32_t *wchunk = nullptr;
   int32_t *zidx = nullptr;
 };
 

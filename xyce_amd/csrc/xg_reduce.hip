@@ -14,11 +14,15 @@
 //    N_DEV_MOSFET_B3.C:9654-9928); padding adds -0.0, the exact identity.
 //  * A segment of at most kChunk sources is folded the same way by one
 //    thread from the contiguous source list.
-//  * A longer segment (a supply rail or a heavily shared node) is folded in
-//    two passes: each chunk is summed in order into a partial, then one
-//    wavefront adds the partials to out[k] in chunk order (lane runs in
-//    lane order).  The order is fixed; the result differs from the strictly
-//    sequential sum by rounding only.
+//  * A longer segment (a supply rail or a heavily shared node) is summed by
+//    chunks: each chunk in order, then one wavefront adds the chunk sums to
+//    out[k] in chunk order (lane runs in lane order).  The order is fixed; the
+//    result differs from the strictly sequential sum by rounding only.  Up to
+//    64 chunks (2048 sources) one wavefront does both, a lane per chunk, in
+//    the same launch; longer ones take two passes, because one wavefront
+//    would walk them behind everything else.  The second launch cost the
+//    101-stage MOSFET1 ring 4.3 us of 22, and every iteration of a batch of
+//    rings 4.8.
 //
 // In the overwrite mode the fold starts from +0.0 instead of out[k] (the
 // same bits as zeroing first) and entries no source reaches are set to
@@ -36,8 +40,9 @@ constexpr int kWaves = kBlock / 64;
 struct ReduceBatch {
   int n;
   int overwrite;
-  // work-item prefixes over the programs: short records, chunks, zero
-  // entries, multi-chunk segments
+  // work-item prefixes over the programs: wide segments (a wavefront each),
+  // short records, chunks, zero entries, multi-chunk segments
+  int32_t wstart[kMaxProgs + 1];
   int32_t s4start[kMaxProgs + 1];
   int32_t sstart[kMaxProgs + 1];
   int32_t cstart[kMaxProgs + 1];
@@ -81,13 +86,61 @@ __device__ __forceinline__ double fold(double acc, const int32_t *__restrict__ s
   return acc;
 }
 
-// One launch for every short record, every chunk and (overwrite mode) every
-// zero entry of all programs, in that order of thread ids, so each wave
-// does one kind of work.
+// The 64 lanes' sums added to r in lane order; each read with readlane (the
+// reads do not wait on the additions, so only the adds are serial).
+__device__ __forceinline__ double add_lanes(double r, double acc) {
+  const long long bits = __double_as_longlong(acc);
+  const int lo = (int)bits, hi = (int)(bits >> 32);
+#pragma unroll
+  for (int l = 0; l < 64; ++l) {
+    const unsigned a = (unsigned)__builtin_amdgcn_readlane(lo, l);
+    const long long h = (long long)__builtin_amdgcn_readlane(hi, l);
+    r = r + __longlong_as_double((long long)((unsigned long long)h << 32 | a));
+  }
+  return r;
+}
+
+// One wide segment: a lane per chunk, every source of a chunk in flight
+// together, then the chunk sums in chunk order.
+__device__ __forceinline__ void fold_wide(const ReduceBatch &b, int w,
+                                          const double *__restrict__ slots) {
+  const int lane = threadIdx.x & 63;
+  const int k = find_prog(b.wstart, b.n, w);
+  const ReduceDev &p = b.prog[k];
+  const int i = w - b.wstart[k];
+  const int32_t t = p.wtgt[i], c0 = p.wchunk[2 * i], c1 = p.wchunk[2 * i + 1];
+  const int32_t c = min(c0 + lane, c1 - 1);
+  const int32_t beg = p.cptr[c], len = c0 + lane < c1 ? p.cptr[c + 1] - beg : 0;
+  int32_t s[kChunk];
+  double v[kChunk];
+#pragma unroll
+  for (int u = 0; u < kChunk; ++u) s[u] = p.src[beg + (u < len ? u : 0)];
+#pragma unroll
+  for (int u = 0; u < kChunk; ++u) v[u] = slots[max(s[u], 0)];
+  double acc = -0.0;
+#pragma unroll
+  for (int u = 0; u < kChunk; ++u) {
+    const double x = acc + (s[u] >= 0 ? v[u] : s[u] == -1 ? 0.0 : -0.0);
+    acc = u < len ? x : acc;
+  }
+  double *out = b.out[k];
+  const double r = add_lanes(b.overwrite ? 0.0 : out[t], acc);
+  if (lane == 0) out[t] = r;
+}
+
+// One launch for every wide segment (the first workgroups), every short
+// record, every chunk and (overwrite mode) every zero entry of all programs,
+// in that order of thread ids, so each wave does one kind of work.
 __global__ void __launch_bounds__(kBlock)
     fold_kernel(ReduceBatch b, const double *__restrict__ slots) {
   if (b.gate && *b.gate) return;
-  int w = blockIdx.x * kBlock + threadIdx.x;
+  const int n_wide = b.wstart[b.n], wblocks = (n_wide + kWaves - 1) / kWaves;
+  if ((int)blockIdx.x < wblocks) {
+    const int w = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    if (w < n_wide) fold_wide(b, w, slots);
+    return;
+  }
+  int w = (blockIdx.x - wblocks) * kBlock + threadIdx.x;
   const int n_short4 = b.s4start[b.n];
   const int n_short = b.sstart[b.n], n_chunk = b.cstart[b.n];
   if (w < n_short4) {
@@ -176,16 +229,7 @@ __global__ void __launch_bounds__(kBlock)
   for (int32_t c = rb; c < re; ++c) acc = acc + b.partial[p.pbase + c];
   double *out = b.out[k];
   double r = b.overwrite ? 0.0 : out[t];
-  // lane runs in lane order; each lane's run sum read with readlane (the
-  // reads do not wait on the additions, so only the adds are serial)
-  const long long bits = __double_as_longlong(acc);
-  const int lo = (int)bits, hi = (int)(bits >> 32);
-#pragma unroll
-  for (int l = 0; l < 64; ++l) {
-    const unsigned a = (unsigned)__builtin_amdgcn_readlane(lo, l);
-    const long long h = (long long)__builtin_amdgcn_readlane(hi, l);
-    r = r + __longlong_as_double((long long)((unsigned long long)h << 32 | a));
-  }
+  r = add_lanes(r, acc);  // lane runs in lane order
   if (lane == 0) out[t] = r;
 }
 
@@ -291,9 +335,11 @@ hipError_t launch_reduce(int n_out, const ReduceDev *progs, double *const *outs,
   for (int k = 0; k < n_out; ++k) {
     b.prog[k] = progs[k];
     b.out[k] = outs[k];
-    const int32_t items = progs[k].n_short4 + progs[k].n_short + progs[k].n_chunk +
+    const int32_t items = progs[k].n_wide + progs[k].n_short4 + progs[k].n_short +
+                          progs[k].n_chunk +
                           (overwrite ? progs[k].n_zero : 0);
     if (!outs[k] && items) return hipErrorInvalidValue;
+    b.wstart[k + 1] = b.wstart[k] + progs[k].n_wide;
     b.s4start[k + 1] = b.s4start[k] + progs[k].n_short4;
     b.sstart[k + 1] = b.sstart[k] + progs[k].n_short;
     b.cstart[k + 1] = b.cstart[k] + progs[k].n_chunk;
@@ -301,6 +347,7 @@ hipError_t launch_reduce(int n_out, const ReduceDev *progs, double *const *outs,
     b.mstart[k + 1] = b.mstart[k] + progs[k].n_multi;
   }
   for (int k = n_out; k < kMaxProgs; ++k) {
+    b.wstart[k + 1] = b.wstart[n_out];
     b.s4start[k + 1] = b.s4start[n_out];
     b.sstart[k + 1] = b.sstart[n_out];
     b.cstart[k + 1] = b.cstart[n_out];
@@ -310,9 +357,11 @@ hipError_t launch_reduce(int n_out, const ReduceDev *progs, double *const *outs,
   const int64_t items = (int64_t)b.s4start[n_out] + b.sstart[n_out] + b.cstart[n_out] +
                         (overwrite ? b.zstart[n_out] : 0);
   const int n_multi = b.mstart[n_out];
-  if (items == 0) return hipSuccess;
-  hipLaunchKernelGGL(fold_kernel, dim3((unsigned)((items + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, s, b, slots);
+  const int64_t wblocks = (b.wstart[n_out] + kWaves - 1) / kWaves;
+  if (items + wblocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(fold_kernel,
+                     dim3((unsigned)(wblocks + (items + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                     s, b, slots);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_multi == 0) return e;
   hipLaunchKernelGGL(combine_kernel, dim3((n_multi + kWaves - 1) / kWaves),

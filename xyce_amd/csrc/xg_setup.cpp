@@ -496,7 +496,18 @@ static void finish_program(const std::vector<Contrib> &cs, int32_t n_out,
   prog.cdst.clear();
   prog.mtgt.clear();
   prog.mchunk.clear();
+  prog.wtgt.clear();
+  prog.wchunk.clear();
   prog.zidx.clear();
+  std::vector<int32_t> wide;
+  auto chunks = [&](int32_t k, int32_t dst) {
+    for (int32_t j = cnt[k]; j < cnt[k + 1]; j += kChunk) {
+      const int32_t e = std::min(cnt[k + 1], j + kChunk);
+      for (int32_t q = j; q < e; ++q) prog.src.push_back(srcs[q]);
+      prog.cptr.push_back((int32_t)prog.src.size());
+      prog.cdst.push_back(dst);
+    }
+  };
   for (int32_t k = 0; k < n_out; ++k) {
     const int32_t len = cnt[k + 1] - cnt[k];
     if (len == 0 || skip[k]) {
@@ -516,17 +527,23 @@ static void finish_program(const std::vector<Contrib> &cs, int32_t n_out,
       continue;
     }
     const int32_t first_chunk = (int32_t)prog.cdst.size();
-    for (int32_t j = cnt[k]; j < cnt[k + 1]; j += kChunk) {
-      const int32_t e = std::min(cnt[k + 1], j + kChunk);
-      for (int32_t q = j; q < e; ++q) prog.src.push_back(srcs[q]);
-      prog.cptr.push_back((int32_t)prog.src.size());
-      prog.cdst.push_back(len <= kChunk ? k : -1);
+    if (len > kChunk && len <= 64 * kChunk) {  // after the others' chunks
+      wide.push_back(k);
+      continue;
     }
+    chunks(k, len <= kChunk ? k : -1);
     if (len > kChunk) {
       prog.mtgt.push_back(k);
       prog.mchunk.push_back(first_chunk);
       prog.mchunk.push_back((int32_t)prog.cdst.size());
     }
+  }
+  prog.n_chunk = (int32_t)prog.cdst.size();
+  for (int32_t k : wide) {
+    prog.wtgt.push_back(k);
+    prog.wchunk.push_back((int32_t)prog.cdst.size());
+    chunks(k, -1);
+    prog.wchunk.push_back((int32_t)prog.cdst.size());
   }
 }
 
