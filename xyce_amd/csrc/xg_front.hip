@@ -233,6 +233,17 @@ __device__ __forceinline__ bool front_skip(const FrontArgs &f, int c) {
   return (f.gate && *f.gate) || (f.active && !f.active[c]) || f.bad[c];
 }
 
+// The same for a workgroup of a launch that sets the flag: another front of
+// component c, in the same launch, can fail while this workgroup's
+// wavefronts start, and wavefronts that read different values would leave some
+// of them running with LDS that the others never wrote.  So one thread reads
+// it for all of them.
+__device__ __forceinline__ bool front_skip_block(const FrontArgs &f, int c, int *flag) {
+  if (threadIdx.x == 0) *flag = front_skip(f, c);
+  __syncthreads();
+  return *flag != 0;
+}
+
 // Clears the fronts and the failure flags and sets the right-hand-side
 // columns, then (second kernel) scatters the Jacobian's entries.
 __global__ void __launch_bounds__(kFB) front_clear_kernel(FrontArgs f, const double *bp) {
@@ -260,10 +271,10 @@ __global__ void __launch_bounds__(BS) front_factor_kernel(FrontArgs f, int lv0) 
   __shared__ double P[ROWS * (NB + 1)];
   __shared__ double sv[BS / 64];
   __shared__ int si[BS / 64];
-  __shared__ int spiv[NB];
+  __shared__ int spiv[NB], skip;
   const int s = f.lv[lv0 + blockIdx.x];
   const int c = f.comp[s];
-  if (front_skip(f, c)) return;
+  if (front_skip_block(f, c, &skip)) return;
   const int t = threadIdx.x;
   const int m = f.m[s], k = f.k[s];
   if (m > f.big_m) return;  // factored by many workgroups (launch_big_front)
@@ -463,6 +474,7 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
   __shared__ double sval[2][4][NW], srcp[2][4][NW], raw[4][W];
   __shared__ int spos[2][4][NW], sphy[2][4][NW], nmove;
   const BigFront s = f.big[lb + blockIdx.x];
+  // (no workgroup of this launch sets f.bad, so every wavefront reads the same)
   if (front_skip(f, s.comp)) return;
   const int m = s.m, k = s.k;
   if (kb >= k) return;
@@ -471,7 +483,8 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
   const int wrow = wave * kRows;
   double *A = f.vals + s.fo + (int64_t)kb * m + kb;
   double *L = f.lbuf + s.lo + kb;  // column c: L + c m
-  if (threadIdx.x == 0) nmove = 0;
+  int32_t *mv = f.mv + (int64_t)blockIdx.x * kMoveInts;
+  if (threadIdx.x == 0) nmove = 0;  // (used behind the columns' barriers)
   double4v acc[kNT][kCT];
 #pragma unroll
   for (int t = 0; t < kNT; ++t)
@@ -564,7 +577,7 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
           best = read_lane(cv, bw);
         }
         if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
-          if (threadIdx.x == 0) f.bad[s.comp] = 1;
+          if (threadIdx.x == 0) mv[0] = -1;  // the solve launch flags the component
           return;
         }
         win |= (unsigned)bw << (4 * j);
@@ -649,7 +662,6 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
     }
   }
   int32_t *piv = f.piv + s.ro + kb;
-  int32_t *mv = f.mv + (int64_t)blockIdx.x * kMoveInts;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = wrow + 64 * q + lane;
@@ -681,7 +693,7 @@ __global__ void __launch_bounds__(64) front_wave_kernel(FrontArgs f, int lv0) {
   __shared__ double raw[4][16 * kCT];
   const int s = f.lv[lv0 + blockIdx.x];
   const int comp = f.comp[s];
-  if (front_skip(f, comp)) return;
+  if (__builtin_amdgcn_readfirstlane(front_skip(f, comp))) return;  // one value for all lanes
   const int m = f.m[s], k = f.k[s];
   if (m > f.big_m) return;  // factored by many workgroups
   const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
@@ -893,7 +905,9 @@ __global__ void __launch_bounds__(64) front_solve_kernel(FrontArgs f, int lb, in
   __shared__ double dr[kBigW];
   __shared__ int32_t top[kBigW], mdst[kBigW], msrc[kBigW];
   const BigFront s = f.big[lb + blockIdx.y];
-  if (front_skip(f, s.comp)) return;
+  // (another front's workgroup may set the flag just now; either value will do,
+  // and this workgroup is one wavefront)
+  if (__builtin_amdgcn_readfirstlane(front_skip(f, s.comp))) return;
   const int m = s.m, k = s.k;
   if (kb >= k) return;
   const int cl = min(kb + wp, k), nw = cl - kb;
@@ -908,6 +922,10 @@ __global__ void __launch_bounds__(64) front_solve_kernel(FrontArgs f, int lb, in
   if (b < ncb) {
     const int32_t *mv = f.mv + (int64_t)blockIdx.y * kMoveInts;
     const int nm = mv[0];
+    if (nm < 0) {  // the panel found no pivot: no rows and no multipliers of it
+      if (b == 0 && lane == 0) f.bad[s.comp] = 1;
+      return;
+    }
     if (lane < kBigW) {  // (padded with readable rows, so no load below is conditional)
       top[lane] = lane < nw ? f.piv[s.ro + kb + lane] : kb;
       mdst[lane] = lane < nm ? mv[1 + 2 * lane] : kb;

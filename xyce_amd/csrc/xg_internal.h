@@ -321,7 +321,7 @@ struct FrontArgs {
   double *vals, *wrhs, *v;        // fronts, front right-hand sides, positions
   int32_t *piv, *bad;             // panel rows before its swaps (at ro), failed components
   // per large front of a launch: the rows a panel's swaps displace from its
-  // block, their number, then (dst, src) pairs
+  // block, their number (-1: the panel found no pivot), then (dst, src) pairs
   int32_t *mv = nullptr;
   // per large front of a level: its panel's multipliers, column c at c m
   double *lbuf = nullptr;
