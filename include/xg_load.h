@@ -414,7 +414,9 @@ int xg_lu_cache_set_limit(int64_t bytes);
    across many workgroups (one workgroup per panel, then every column's row
    swaps and U12 rows and the rows below, then the trailing update in 64 x 64
    tiles); smaller ones by one wavefront or workgroup each.  All forms give
-   the same bits.  No counterpart in the reference (tuning and tests). */
+   the same bits.  Takes effect on solves enqueued afterwards; captured graphs
+   (a transient driver's, too) keep the threshold they were captured with.
+   No counterpart in the reference (tuning and tests). */
 int xg_lu_front_set_big(xg_handle *h, int32_t big_m);
 
 /* Components too large for the task lists of xg_lu_info (more than 4 M

@@ -292,3 +292,37 @@ def test_fronts_pivot_on_random_values_without_fallback(big_m):
     assert x1.tobytes() == x.tobytes()
     fr.close()
 
+
+
+def test_threshold_change_leaves_captured_graphs_alone():
+    """xg_lu_front_set_big after a transient driver captured its graphs: the
+    graphs go on with the fronts, launch sizes and panel buffers they were
+    captured with, whatever thresholds follow, and solves enqueued in between
+    take theirs -- all with the same bits."""
+    import torch
+    from xyce_amd import circuits
+    from xyce_amd._lib import check, lib
+    from xyce_amd.transient import Transient
+
+    def run(change):
+        tr = Transient(circuits.random_logic_bsim3(n_gates=300, seed=8, ramp=50e-12),
+                       lu_fronts=True)
+        fp = tr.dev.front_plan()
+        # the thresholds below part the fronts differently
+        assert len({int((fp["m"] > b).sum()) for b in (64, 1, 8, 40, 1 << 30)}) == 5
+        rng = np.random.default_rng(3)
+        nnz, n1 = tr.dev.nnz, tr.dev.n_rows
+        rows = np.repeat(np.arange(n1), np.diff(tr.dev.pattern()[0]))
+        vals = rng.standard_normal(nnz) + 20.0 * (rows == tr.dev.pattern()[1])
+        rhs = np.append(rng.standard_normal(n1 - 1), 0.0)
+        out = []
+        for big_m in (64, 1, 1 << 30, 8, 40, 1):
+            if change:
+                check(lib().xg_lu_front_set_big(tr.dev.h, big_m), "front threshold")
+            t, w = tr.run(20e-12, 1e-12, ["g0", "g1"], uic=True)
+            out += [w, tr.x_curr.cpu().numpy().copy(), _solve(tr.dev, vals, rhs, torch)[0]]
+        tr.close()
+        return out
+
+    for a, b in zip(run(True), run(False)):
+        assert a.tobytes() == b.tobytes()

@@ -29,6 +29,14 @@ struct DevBuf {
   }
 };
 
+// A plan's fronts above some number of rows, by level: level l's are
+// [ptr[l], ptr[l + 1]), on the host and on the device.
+struct BigList {
+  std::vector<BigFront> big;
+  std::vector<int32_t> ptr;
+  BigFront *dev = nullptr;
+};
+
 struct Handle {
   Plan plan;
   hipStream_t stream = nullptr;
@@ -48,10 +56,11 @@ struct Handle {
   SparseLuArgs lu{};
   FrontArgs fr{};
   std::vector<int32_t> fr_lv, fr_cls, fr_lv_maxm;  // host copies for the launches
-  // fronts of more than fr.big_m rows by level (host, offsets, device)
-  std::vector<BigFront> fr_big;
-  std::vector<int32_t> fr_big_ptr;
-  BigFront *fr_big_dev = nullptr;
+  // the fronts of more than fr.big_m rows: one list per number of them, kept
+  // until the handle goes (a captured graph holds the list that it was
+  // captured with, its launch sizes and its panel buffers)
+  std::map<size_t, BigList> fr_lists;
+  const BigList *fr_big = nullptr;
   int32_t fr_mv_n = 0;    // large fronts that fr.mv has room for
   int64_t fr_lbuf_n = 0;  // doubles in fr.lbuf
   std::vector<int64_t> fr_xr_off;  // receiving rows per front (host copy)
@@ -494,9 +503,9 @@ int xg_lu_solve(xg_handle *H, const double *J, const double *rhs, double *x,
     const xg::LuPlan &L = h.plan.lu;
     f.lv_host = h.fr_lv.data();
     f.m_host = L.fr_m.data();
-    f.big = h.fr_big_dev;
-    f.big_host = h.fr_big.data();
-    f.big_ptr_host = h.fr_big_ptr.data();
+    f.big = h.fr_big->dev;
+    f.big_host = h.fr_big->big.data();
+    f.big_ptr_host = h.fr_big->ptr.data();
     e = xg::launch_fronts(f, u, h.stream);
     if (e != hipSuccess) return hip_fail(e, "front LU");
   }
@@ -547,45 +556,47 @@ int xg_lu_info(xg_handle *H, int64_t *info) {
   return XG_OK;
 }
 
-// The fronts of more than big_m rows grouped by level, on the host and (once
-// uploaded) on the device.
-static int front_big_lists(xg::Handle &h) {
+// Makes the fronts of more than big_m rows the handle's large ones.  Nothing
+// of an earlier list is overwritten or freed: work in flight and captured
+// graphs go on with theirs.  On a failure the handle keeps what it had.
+static int front_big_lists(xg::Handle &h, int32_t big_m) {
   const xg::LuPlan &L = h.plan.lu;
-  h.fr_big.clear();
-  h.fr_big_ptr.assign(1, 0);
+  xg::BigList n;
+  n.ptr.push_back(0);
   int32_t most = 0;     // of a level
   int64_t most_lo = 0;  // panel buffers of a level
   for (size_t l = 0; l + 1 < L.fr_lv_ptr.size(); ++l) {
     int64_t lo = 0;
-    for (int32_t q = L.fr_lv_ptr[l]; q < L.fr_lv_ptr[l + 1]; ++q)
-      if (L.fr_m[L.fr_lv[q]] > h.fr.big_m) {
-        const int32_t s = L.fr_lv[q];
-        const bool have = !h.fr_xr_off.empty();
-        h.fr_big.push_back({L.fr_fo[s], L.fr_ro[s], have ? h.fr_xr_off[s] : 0,
-                            have ? h.fr_xr_off[s + 1] : 0, lo, L.fr_m[s], L.fr_k[s],
-                            L.fr_comp[s], s});
-        lo += (int64_t)xg::kBigW * L.fr_m[s];
-      }
+    for (int32_t q = L.fr_lv_ptr[l]; q < L.fr_lv_ptr[l + 1]; ++q) {
+      const int32_t s = L.fr_lv[q];
+      if (L.fr_m[s] <= big_m) continue;
+      n.big.push_back({L.fr_fo[s], L.fr_ro[s], h.fr_xr_off[s], h.fr_xr_off[s + 1], lo,
+                       L.fr_m[s], L.fr_k[s], L.fr_comp[s], s});
+      lo += (int64_t)xg::kBigW * L.fr_m[s];
+    }
     most_lo = std::max(most_lo, lo);
-    most = std::max(most, (int32_t)h.fr_big.size() - h.fr_big_ptr.back());
-    h.fr_big_ptr.push_back((int32_t)h.fr_big.size());
+    most = std::max(most, (int32_t)n.big.size() - n.ptr.back());
+    n.ptr.push_back((int32_t)n.big.size());
   }
   most = std::min(most, (int32_t)xg::kBigLaunch);
-  // (earlier, smaller buffers live on: a captured graph may hold them)
-  if (h.fr_big_dev && most > h.fr_mv_n) {
-    h.fr.mv = h.alloc<int32_t>((size_t)most * xg::kMoveInts);
-    if (!h.fr.mv) return XG_E_NOMEM;
-    h.fr_mv_n = most;
+  // (thresholds with as many fronts above them have the same list)
+  auto it = h.fr_lists.find(n.big.size());
+  if (it == h.fr_lists.end()) {
+    int32_t *mv = h.fr.mv;
+    double *lbuf = h.fr.lbuf;
+    if (most > h.fr_mv_n) mv = h.alloc<int32_t>((size_t)most * xg::kMoveInts);
+    if (most_lo > h.fr_lbuf_n) lbuf = h.alloc<double>((size_t)most_lo);
+    n.dev = h.upload(n.big);
+    if ((most && (!mv || !lbuf)) || !n.dev) return XG_E_NOMEM;
+    h.fr.mv = mv;
+    h.fr.lbuf = lbuf;
+    h.fr_mv_n = std::max(h.fr_mv_n, most);
+    h.fr_lbuf_n = std::max(h.fr_lbuf_n, most_lo);
+    const size_t key = n.big.size();
+    it = h.fr_lists.emplace(key, std::move(n)).first;
   }
-  if (h.fr_big_dev && most_lo > h.fr_lbuf_n) {
-    h.fr.lbuf = h.alloc<double>((size_t)most_lo);
-    if (!h.fr.lbuf) return XG_E_NOMEM;
-    h.fr_lbuf_n = most_lo;
-  }
-  if (h.fr_big_dev && !h.fr_big.empty() &&
-      hipMemcpy(h.fr_big_dev, h.fr_big.data(), sizeof(xg::BigFront) * h.fr_big.size(),
-                hipMemcpyHostToDevice) != hipSuccess)
-    return XG_E_HIP;
+  h.fr_big = &it->second;
+  h.fr.big_m = big_m;
   return XG_OK;
 }
 
@@ -603,8 +614,11 @@ int xg_lu_cache_set_limit(int64_t bytes) {
 
 int xg_lu_front_set_big(xg_handle *H, int32_t big_m) {
   if (!H || big_m < 1) return fail(XG_E_ARG, "xg_lu_front_set_big");
-  H->h.fr.big_m = big_m;
-  if (front_big_lists(H->h)) return fail(XG_E_HIP, "xg_lu_front_set_big: upload");
+  if (H->h.plan_only || H->h.fr.n_fronts == 0) {  // no lists on a device (yet)
+    H->h.fr.big_m = big_m;
+    return XG_OK;
+  }
+  if (front_big_lists(H->h, big_m)) return fail(XG_E_HIP, "xg_lu_front_set_big: upload");
   return XG_OK;
 }
 
@@ -1067,8 +1081,10 @@ static bool upload_handle(xg_handle *H) {
           xr_off[s + 1] = (int64_t)xr_row.size();
         }
         h.fr_xr_off = xr_off;
-        chk(h.fr_big_dev = h.alloc<xg::BigFront>((size_t)nf));
-        if (ok && front_big_lists(h)) ok = false;
+        h.fr_lists.clear();
+        h.fr_mv_n = 0;
+        h.fr_lbuf_n = 0;
+        if (ok && front_big_lists(h, f.big_m)) ok = false;
         chk(f.xr_row = h.upload(xr_row));
         chk(f.ext_ptr = h.upload(ext_ptr));
         chk(f.ext_ch = h.upload(ext_ch));
