@@ -395,11 +395,20 @@ struct CompLu {
 // ones), a column step of a front ~1 us.  So the deepest children of a front
 // join it together (a part of them would leave the height as it is) while the
 // columns that this makes serial -- all but the longest child's -- cost less
-// than the level: kMergeSmall of them up to kMergeRows rows, kMergeBig above,
-// where the zeros stored may cost kMergeFlops (~10 us).  A front does not
-// outgrow a wavefront this way, except with a child that adds no zeros.  5,000-gate logic: 18,215 fronts in 26 levels
-// before.
-constexpr int64_t kMergeRows = 64, kMergeSmall = 8, kMergeBig = 24, kMergeFlops = 30000000;
+// than the level: kMergeSmall of them up to kMergeSmallRows rows, none up to
+// kMergeRows, kMergeBig above, where the zeros stored may cost kMergeFlops
+// (~10 us).  A front does not outgrow a wavefront this way, except with a
+// child that adds no zeros.
+//
+// The limits are also the solution's precision.  A joined child's columns are
+// subtracted group by group from entries of full size; as a front of its own
+// it sums them from zero and adds the sum once.  On power grids, whose rows
+// nearly cancel, eight columns up to 64 rows instead of 24 took 1.2 times the
+// error (28 x 28 mesh: 1.7e-15 against 1.35e-15; no joining at all: 1.26e-15 with
+// one chain per entry).  5,000-gate logic: 18,215 fronts in 26 levels without,
+// 5 levels with; 100 x 100 grid 34 levels and 6, 10,000-node ladder 23 and 4.
+constexpr int64_t kMergeRows = 64, kMergeSmallRows = 24, kMergeSmall = 8, kMergeBig = 16,
+                  kMergeFlops = 30000000;
 
 std::vector<std::vector<int32_t>> front_tree(int32_t n, const std::vector<int32_t> &parent,
                                              const std::vector<std::vector<int32_t>> &ucol) {
@@ -428,9 +437,10 @@ std::vector<std::vector<int32_t>> front_tree(int32_t n, const std::vector<int32_
           parts += cost(kc + (int64_t)ucol[c].size(), kc);
         }
       const bool small = m + sum <= kMergeRows;
+      const int64_t serial = m + sum <= kMergeSmallRows ? kMergeSmall : small ? 0 : kMergeBig;
       if (m + sum > kFrontMaxM) break;
       if (!same && ((m <= kMergeRows && !small) ||
-                    sum - most > (small ? kMergeSmall : kMergeBig) ||
+                    sum - most > serial ||
                     (!small && cost(m + sum, k + sum) - parts > (double)kMergeFlops)))
         break;
       std::vector<int32_t> left;
