@@ -74,3 +74,60 @@ def test_front_forms_at_their_edges(n, extra):
     for x in out[1:]:
         assert x.tobytes() == out[0].tobytes()
     dev.close()
+
+
+def _random_graph(n, degree):
+    """n nodes, each joined to `degree` earlier ones at random: the last front
+    takes most of them."""
+    from xyce_amd import circuits
+    rng = np.random.default_rng(1)
+    nl = circuits.Netlist("random graph")
+    for i in range(1, n):
+        for j in rng.integers(0, i, min(degree, i)):
+            nl.add_res("R%d" % len(nl.res), "n%d" % i, "n%d" % int(j), 1.0)
+    nl.add_res("R%d" % len(nl.res), "n0", "0", 1.0)
+    return nl.layout()
+
+
+# the panel's classes above the cliques': 1024 and 2048 fully summed rows, with
+# a root just above each and one near the largest front's
+@pytest.mark.parametrize("n,degree,low,high", [(2500, 5, 1024, 1200), (2900, 16, 2048, 2200),
+                                               (4100, 20, 3400, 3481)])
+def test_tall_panels(n, degree, low, high):
+    import torch
+    from xyce_amd._lib import check, lib
+    from xyce_amd.loader import DeviceLoad, _ptr
+    nl = _random_graph(n, degree)
+    dev = DeviceLoad(nl, lu_fronts=True)
+    root = int(dev.front_plan()["k"].max())
+    print("case: random graph of", n, "largest front", root, flush=True)
+    assert low < root <= high
+    rp, ci = dev.pattern()
+    rows = np.repeat(np.arange(n + 1), np.diff(rp))
+    keep = (rows < n) & (ci < n)
+    r, c = rows[keep], ci[keep]
+    rng = np.random.default_rng(n)
+    vals = rng.standard_normal(len(ci)) + 2.0 * (rows == ci)
+    rhs = np.append(rng.standard_normal(n), 0.0)
+    v = vals[keep]
+    nc = ctypes.c_int32()
+    check(lib().xg_components(dev.h, ctypes.byref(nc), None), "components")
+    cu = lambda q: torch.tensor(q, dtype=torch.float64, device="cuda")
+    out = []
+    for big_m in (64, 1 << 30):
+        check(lib().xg_lu_front_set_big(dev.h, big_m), "set big")
+        J, R, X, W = cu(vals), cu(rhs), cu(np.zeros(n + 1)), cu(np.ones(n + 1))
+        st = cu(np.zeros(4 * nc.value))
+        check(lib().xg_lu_solve(dev.h, _ptr(J), _ptr(R), _ptr(X), _ptr(W), _ptr(W), 0.0, 1.0,
+                                None, _ptr(st)), "lu solve")
+        dev.sync()
+        x = X.cpu().numpy()[:n]
+        print("threshold", big_m, flush=True)
+        assert not st.cpu().numpy().reshape(-1, 4)[:, 2].any()
+        ax = np.bincount(r, v * x[c], n)
+        berr = np.abs(ax - rhs[:n]).max() / (np.bincount(r, np.abs(v), n).max() * np.abs(x).max() +
+                                             np.abs(rhs[:n]).max())
+        assert berr < 1e-12   # the bound the solve itself accepts
+        out.append(x)
+    assert out[1].tobytes() == out[0].tobytes()
+    dev.close()

@@ -40,3 +40,13 @@ def test_fold_keeps_full_occupancy():
     for name, r in folds.items():
         assert r["Occupancy [waves/SIMD]"] == 8, (name, r)
         assert r["SGPRs Spill"] == 0 and r["VGPRs Spill"] == 0, (name, r)
+
+
+def test_panels_spill_no_register():
+    """A panel's row tiles are in registers (or its rows in memory, above 2048)
+    so that a column step waits on its own chain only."""
+    panels = {k: v for k, v in _report("xg_front.hip").items() if "panel_kernel" in k}
+    assert len(panels) == 6
+    for name, r in panels.items():
+        assert r["VGPRs Spill"] == 0, (name, r)
+        assert r["ScratchSize [bytes/lane]"] == 0, (name, r)

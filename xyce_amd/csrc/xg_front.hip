@@ -530,15 +530,137 @@ __device__ __forceinline__ double4v add_group(double a, double b, const double4v
   return {acc[0] + p[0], acc[1] + p[1], acc[2] + p[2], acc[3] + p[3]};
 }
 
+// What a panel's wavefronts exchange in a group of four columns: their
+// candidates (value, reciprocal, position, row) and candidate rows' entries of
+// these columns, two groups deep.
+template <int NW>
+struct PanelLds {
+  double srow[2][4][NW][4];
+  double sval[2][4][NW], srcp[2][4][NW];
+  int spos[2][4][NW], sphy[2][4][NW], nmove;
+};
+
+// The column steps of one group, a row's entries of its four columns per lane
+// (a; R rows each, at positions pos): ln gets minus the multipliers, L their
+// columns, A the pivot rows' entries, win each pivot row's wavefront (four
+// bits each).  False when a column has no pivot.
+template <int NW, int R>
+__device__ __forceinline__ bool panel_columns(PanelLds<NW> &sh, int par, int c0, int nw, int wrow,
+                                              double (&a)[R][4], double (&ln)[R][4],
+                                              int (&pos)[R], double *A, double *L, int m,
+                                              int32_t *mv, unsigned &win) {
+  constexpr int kSteps = NW >= 16 ? 4 : NW >= 8 ? 3 : NW >= 4 ? 2 : 1;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  win = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int c = c0 + j;
+    if (c >= nw) continue;
+    double v = 0.0, x0 = 0.0;
+    int p = 0x7fffffff, qb = 0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double x = fabs(a[q][j]);
+      if (pos[q] >= c && (x > v || (x == v && pos[q] < p))) {
+        v = x;
+        x0 = a[q][j];
+        p = pos[q];
+        qb = q;
+      }
+    }
+    // the reciprocal every lane's candidate would need, while the
+    // search below waits on its chain
+    double rcp = make_pivot(x0).r;
+    const int wl = lane_of_max<6>(v, p);
+    if (lane == wl) {
+      sh.sval[par][j][wave] = v;
+      sh.srcp[par][j][wave] = rcp;
+      sh.spos[par][j][wave] = p;
+      sh.sphy[par][j][wave] = wrow + 64 * qb + lane;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        double x = a[0][jj];
+#pragma unroll
+        for (int q = 1; q < R; ++q) {
+          double aq = a[q][jj];
+          asm("" : "+v"(aq));  // a select of values, not an indexed load
+          x = qb == q ? aq : x;
+        }
+        sh.srow[par][j][wave][jj] = x;
+      }
+    }
+    int bw = 0;
+    double best;
+    if constexpr (NW == 1) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      best = sh.sval[par][j][0];
+    } else {
+      __syncthreads();
+      // the best wavefront: lanes 0..NW-1 hold the candidates
+      const double cv = lane < NW ? sh.sval[par][j][lane] : 0.0;
+      const int cp = lane < NW ? sh.spos[par][j][lane] : 0x7fffffff;
+      bw = lane_of_max<kSteps>(cv, cp);
+      best = read_lane(cv, bw);
+    }
+    if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
+      if (threadIdx.x == 0) mv[0] = -1;  // the solve launch flags the component
+      return false;
+    }
+    win |= (unsigned)bw << (4 * j);
+    const int bp = sh.spos[par][j][bw];
+    double u[4];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) u[jj] = sh.srow[par][j][bw][jj];
+    const Pivot pv{__builtin_amdgcn_frexp_mant(u[j]), sh.srcp[par][j][bw],
+                   -__builtin_amdgcn_frexp_exp(u[j])};
+    // the finished pivot row's entries of these columns
+    if (wave == 0 && lane >= j && lane < 4 && c0 + lane < nw)
+      A[(int64_t)c * m + c0 + lane] = sh.srow[par][j][bw][lane];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      pos[q] = pos[q] == bp ? c : (pos[q] == c ? bp : pos[q]);
+      if (pos[q] > c) {
+        const double l = divide(a[q][j], pv);
+        L[(int64_t)c * m + wrow + 64 * q + lane] = l;
+        a[q][j] = l;
+        ln[q][j] = -l;
+#pragma unroll
+        for (int jj = j + 1; jj < 4; ++jj) a[q][jj] = fma(-l, u[jj], a[q][jj]);
+      }
+    }
+  }
+  return true;
+}
+
+// The rows at each position after a panel, and those displaced from its block.
+template <int NW, int R>
+__device__ __forceinline__ void panel_rows(PanelLds<NW> &sh, const int (&pos)[R], int wrow,
+                                           int nw, int kb, int32_t *piv, int32_t *mv) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int r = wrow + 64 * q + lane;
+    if (pos[q] >= 0) {
+      piv[pos[q]] = kb + r;
+      if (pos[q] >= nw && pos[q] != r) {
+        const int e = atomicAdd(&sh.nmove, 1);  // at most nw rows
+        mv[1 + 2 * e] = kb + pos[q];
+        mv[2 + 2 * e] = kb + r;
+      }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) mv[0] = sh.nmove;
+}
+
 template <int NW, int kNT, int kCT>
 __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int lb, int kb) {
   constexpr int R = kNT / 4, W = 16 * kCT, kRows = 16 * kNT;
   static_assert(kNT % 4 == 0 && NW <= 16 && (NW & (NW - 1)) == 0, "rows per lane, search");
-  constexpr int kSteps = NW >= 16 ? 4 : NW >= 8 ? 3 : NW >= 4 ? 2 : 1;
   __shared__ __align__(16) double S[NW][kRows][4];
-  __shared__ __align__(16) double srow[2][4][NW][4];
-  __shared__ double sval[2][4][NW], srcp[2][4][NW], raw[4][W];
-  __shared__ int spos[2][4][NW], sphy[2][4][NW], nmove;
+  __shared__ __align__(16) PanelLds<NW> sh;
+  __shared__ double raw[4][W];
   const BigFront s = f.big[lb + blockIdx.x];
   // (no workgroup of this launch sets f.bad, so every wavefront reads the same)
   if (front_skip(f, s.comp)) return;
@@ -550,7 +672,7 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
   double *A = f.vals + s.fo + (int64_t)kb * m + kb;
   double *L = f.lbuf + s.lo + kb;  // column c: L + c m
   int32_t *mv = f.mv + (int64_t)blockIdx.x * kMoveInts;
-  if (threadIdx.x == 0) nmove = 0;  // (used behind the columns' barriers)
+  if (threadIdx.x == 0) sh.nmove = 0;  // (used behind the columns' barriers)
   double4v acc[kNT][kCT];
 #pragma unroll
   for (int t = 0; t < kNT; ++t)
@@ -590,91 +712,14 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
           a[q][j] = S[wave][64 * q + lane][j];
           ln[q][j] = -0.0;
         }
-      unsigned win = 0;  // the wavefront of each pivot row, four bits each
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = c0 + j;
-        if (c >= nw) continue;
-        double v = 0.0, x0 = 0.0;
-        int p = 0x7fffffff, qb = 0;
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const double x = fabs(a[q][j]);
-          if (pos[q] >= c && (x > v || (x == v && pos[q] < p))) {
-            v = x;
-            x0 = a[q][j];
-            p = pos[q];
-            qb = q;
-          }
-        }
-        // the reciprocal every lane's candidate would need, while the
-        // search below waits on its chain
-        double rcp = make_pivot(x0).r;
-        const int wl = lane_of_max<6>(v, p);
-        if (lane == wl) {
-          sval[par][j][wave] = v;
-          srcp[par][j][wave] = rcp;
-          spos[par][j][wave] = p;
-          sphy[par][j][wave] = wrow + 64 * qb + lane;
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            double x = a[0][jj];
-#pragma unroll
-            for (int q = 1; q < R; ++q) {
-              double aq = a[q][jj];
-              asm("" : "+v"(aq));  // a select of values, not an indexed load
-              x = qb == q ? aq : x;
-            }
-            srow[par][j][wave][jj] = x;
-          }
-        }
-        int bw = 0;
-        double best;
-        if constexpr (NW == 1) {
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          best = sval[par][j][0];
-        } else {
-          __syncthreads();
-          // the best wavefront: lanes 0..NW-1 hold the candidates
-          const double cv = lane < NW ? sval[par][j][lane] : 0.0;
-          const int cp = lane < NW ? spos[par][j][lane] : 0x7fffffff;
-          bw = lane_of_max<kSteps>(cv, cp);
-          best = read_lane(cv, bw);
-        }
-        if (!(best > 0.0) || !(best <= DBL_MAX)) {  // the same in every lane
-          if (threadIdx.x == 0) mv[0] = -1;  // the solve launch flags the component
-          return;
-        }
-        win |= (unsigned)bw << (4 * j);
-        const int bp = spos[par][j][bw];
-        double u[4];
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) u[jj] = srow[par][j][bw][jj];
-        const Pivot pv{__builtin_amdgcn_frexp_mant(u[j]), srcp[par][j][bw],
-                       -__builtin_amdgcn_frexp_exp(u[j])};
-        // the finished pivot row's entries of these columns
-        if (wave == 0 && lane >= j && lane < 4 && c0 + lane < nw)
-          A[(int64_t)c * m + c0 + lane] = srow[par][j][bw][lane];
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          pos[q] = pos[q] == bp ? c : (pos[q] == c ? bp : pos[q]);
-          if (pos[q] > c) {
-            const double l = divide(a[q][j], pv);
-            L[(int64_t)c * m + wrow + 64 * q + lane] = l;
-            a[q][j] = l;
-            ln[q][j] = -l;
-#pragma unroll
-            for (int jj = j + 1; jj < 4; ++jj) a[q][jj] = fma(-l, u[jj], a[q][jj]);
-          }
-        }
-      }
+      unsigned win;  // the wavefront of each pivot row, four bits each
+      if (!panel_columns(sh, par, c0, nw, wrow, a, ln, pos, A, L, m, mv, win)) return;
       if (c0 + 4 >= nw) break;
       // the four pivot rows' other columns, from the lanes that hold them
 #pragma unroll 1
       for (int j = 0; j < 4; ++j) {
         const int ph =
-            __builtin_amdgcn_readfirstlane(sphy[par][j][win >> (4 * j) & 15]) - wrow;
+            __builtin_amdgcn_readfirstlane(sh.sphy[par][j][win >> (4 * j) & 15]) - wrow;
         if (ph < 0 || ph >= kRows) continue;
 #pragma unroll
         for (int t = 0; t < kNT; ++t)
@@ -703,7 +748,7 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
         for (int j = 0; j < 4; ++j) {
           u[j] = raw[j][16 * q + li];
 #pragma unroll
-          for (int i = 0; i < j; ++i) u[j] = fma(-srow[par][j][win >> (4 * j) & 15][i], u[i], u[j]);
+          for (int i = 0; i < j; ++i) u[j] = fma(-sh.srow[par][j][win >> (4 * j) & 15][i], u[i], u[j]);
         }
         const int col = 16 * q + li;
         const double x = lk == 0 ? u[0] : lk == 1 ? u[1] : lk == 2 ? u[2] : u[3];
@@ -727,21 +772,96 @@ __global__ void __launch_bounds__(NW * 64) front_panel_kernel(FrontArgs f, int l
       __builtin_amdgcn_wave_barrier();
     }
   }
-  int32_t *piv = f.piv + s.ro + kb;
+  panel_rows(sh, pos, wrow, nw, kb, f.piv + s.ro + kb, mv);
+}
+
+// The same for more rows than the registers hold (above 2048): the panel's 16
+// columns wait in the panel buffer, a column's place until its multipliers
+// take it, and a group's products are added to them there, a row per lane.
+// In registers, 28 row tiles a wavefront, the compiler spilled 319 of them: a
+// 3440-row front took 26.5 ms, here 20.9.
+template <int NW, int R>
+__global__ void __launch_bounds__(NW * 64) front_tall_panel_kernel(FrontArgs f, int lb, int kb) {
+  constexpr int W = 16;
+  static_assert(kFrontMaxM <= NW * 64 * R, "rows of the tallest panel");
+  __shared__ __align__(16) PanelLds<NW> sh;
+  __shared__ double U[4][W];
+  const BigFront s = f.big[lb + blockIdx.x];
+  // (no workgroup of this launch sets f.bad, so every wavefront reads the same)
+  if (front_skip(f, s.comp)) return;
+  const int m = s.m, k = s.k;
+  if (kb >= k) return;
+  const int nw = min(W, k - kb), nr = k - kb;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wrow = wave * 64 * R;
+  double *A = f.vals + s.fo + (int64_t)kb * m + kb;
+  double *L = f.lbuf + s.lo + kb;  // column c: L + c m
+  int32_t *mv = f.mv + (int64_t)blockIdx.x * kMoveInts;
+  if (threadIdx.x == 0) sh.nmove = 0;  // (used behind the columns' barriers)
+  int pos[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = wrow + 64 * q + lane;
-    if (pos[q] >= 0) {
-      piv[pos[q]] = kb + r;
-      if (pos[q] >= nw && pos[q] != r) {
-        const int e = atomicAdd(&nmove, 1);  // at most nw rows
-        mv[1 + 2 * e] = kb + pos[q];
-        mv[2 + 2 * e] = kb + r;
+    pos[q] = r < nr ? r : -1;
+  }
+  // rows of A to the buffer's columns, a quarter wavefront along a row
+  {
+    const int li = lane & 15;
+#pragma unroll 4
+    for (int r = wrow + (lane >> 4); r < min(wrow + 64 * R, nr); r += 4)
+      if (li < nw) L[(int64_t)li * m + r] = A[(int64_t)r * m + li];
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int c0 = 0; c0 < nw; c0 += 4) {
+    const int par = (c0 >> 2) & 1;
+    double a[R][4], ln[R][4];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        a[q][j] = load_if((pos[q] >= 0) & (c0 + j < nw), L,
+                          (int64_t)(c0 + j) * m + wrow + 64 * q + lane);
+        ln[q][j] = -0.0;
+      }
+    unsigned win;
+    if (!panel_columns(sh, par, c0, nw, wrow, a, ln, pos, A, L, m, mv, win)) return;
+    const int nc = nw - c0 - 4;  // the columns after the group
+    if (nc <= 0) break;
+    // the four pivot rows' entries of them (complete: the columns' barriers
+    // lie behind the last group's sums), a column per lane
+    if (threadIdx.x < nc) {
+      const int col = c0 + 4 + threadIdx.x;
+      double u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        u[j] = L[(int64_t)col * m + sh.sphy[par][j][win >> (4 * j) & 15]];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int i = 0; i < j; ++i)
+          u[j] = fma(-sh.srow[par][j][win >> (4 * j) & 15][i], u[i], u[j]);
+        U[j][threadIdx.x] = u[j];
+        A[(int64_t)(c0 + j) * m + col] = u[j];
+      }
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int c = 0; c < nc; ++c) {
+      double *Lc = L + (int64_t)(c0 + 4 + c) * m + wrow + lane;
+      double x[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) x[q] = load_if(pos[q] > c0 + 3, Lc, 64 * q);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        double p = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p = fma(ln[q][j], U[j][c], p);
+        if (pos[q] > c0 + 3) Lc[64 * q] = x[q] + p;
       }
     }
   }
-  __syncthreads();
-  if (threadIdx.x == 0) mv[0] = nmove;
+  panel_rows(sh, pos, wrow, nw, kb, f.piv + s.ro + kb, mv);
 }
 
 // One wavefront per front of up to 64 rows: the front and its right-hand
@@ -1516,7 +1636,8 @@ hipError_t launch_level(const FrontArgs &f, int lv0, int nfr, hipStream_t s) {
 
 // The panel launch for `nr` fully summed rows left, its width: 32 columns
 // while a lane holds at most two rows, so that the tiles fit the registers of
-// eight wavefronts (256 a lane), 16 above.
+// eight wavefronts (256 a lane), 16 above; from 2048 rows on they wait in
+// memory.
 int launch_panel(const FrontArgs &f, int lb, int nb, int kb, int nr, hipStream_t s) {
 #define XG_PANEL(NW, NT, CT)                                                             \
   do {                                                                                   \
@@ -1529,9 +1650,9 @@ int launch_panel(const FrontArgs &f, int lb, int nb, int kb, int nr, hipStream_t
   if (nr <= 512) XG_PANEL(8, 4, 2);
   if (nr <= 1024) XG_PANEL(8, 8, 2);
   if (nr <= 2048) XG_PANEL(8, 16, 1);
-  static_assert(kFrontMaxM <= 8 * 16 * 28, "rows of the widest panel form");
-  XG_PANEL(8, 28, 1);
 #undef XG_PANEL
+  hipLaunchKernelGGL((front_tall_panel_kernel<8, 7>), dim3(nb), dim3(64 * 8), 0, s, f, lb, kb);
+  return 16;
 }
 
 // A level's fronts of more than big_m rows (f.big[lb, lb + nb)) by many
