@@ -1714,8 +1714,9 @@ hipError_t launch_fronts(const FrontArgs &f, const SparseLuArgs &a, hipStream_t 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   for (int L = 0; L < f.n_levels; ++L) {
-    // the level's fronts by size class (kTinyM rows, 64 rows, larger): the
-    // first by threads, the others up to big_m rows by a workgroup each
+    // the level's fronts by size class (kTinyM rows, 64 rows, larger): those
+    // up to 64 rows by threads and wavefronts, larger ones up to big_m rows
+    // (when that is raised) by a workgroup each, the rest by many
     const int32_t *cp = f.cls_host + 3 * L;
     const int lv0 = cp[0], mid0 = cp[1], big0 = cp[2], lv1 = cp[3];
     int32_t one_max = 0;  // largest of the last class up to big_m rows

@@ -31,6 +31,9 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kLdsBytes = 144 * 1024;  // factors, vector and task lists
+// A component is in LDS when its lists fit at 16 bytes a task and 8 an op
+// (sparse_lu_lds_bytes), so none of its numbers exceeds this, and the packed
+// lists hold each in 16 bits, a divisor with its sign.
 static_assert(kLdsBytes / 8 < 32768, "packed task lists hold 15-bit numbers");
 
 __device__ __forceinline__ double blk_max(double v, double *sv) {
@@ -70,8 +73,7 @@ struct Task {
 // The task lists of one component, level pointers relative to `tasks`.  In
 // LDS (kLds) tasks and ops are packed into 8 and 4 bytes (SparseLuArgs::
 // ptasks, pops): half the bytes to stage on every solve and one LDS word per
-// op.  Every number of a component that fits in LDS fits in 15 bits (144 KB
-// hold at most 18,432 values or ops).
+// op.
 template <bool kLds>
 struct Lists {
   using RawTask = std::conditional_t<kLds, uint2, int4>;
@@ -449,6 +451,10 @@ __global__ void __launch_bounds__(kBlock) sparse_lu_kernel(SparseLuArgs a) {
 
 }  // namespace
 
+// The lists count at their unpacked size: twice what the kernel lays out, so
+// that the packed numbers fit (above).  Components between the two counts
+// take the fronts or the lists in global memory; whether the packed lists in
+// LDS would be faster there has not been measured.
 int64_t sparse_lu_lds_bytes(int64_t n, int64_t fnnz, int64_t tasks, int64_t ops,
                             int64_t levels) {
   return align16(fnnz * 8) + align16(n * 8) + tasks * 16 + align16(ops * 8) +
