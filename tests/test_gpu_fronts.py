@@ -310,8 +310,8 @@ def test_threshold_change_leaves_captured_graphs_alone():
         fp = tr.dev.front_plan()
         # the thresholds below part the fronts differently
         m = np.unique(fp["m"])
-        thresholds = [64, 1, 1 << 30, 8, int(m[-2]), 1]
-        assert len({int((fp["m"] > b).sum()) for b in thresholds}) == 5
+        thresholds = [64, 1, 1 << 30, 8, int(m[len(m) // 2]), 1]
+        assert len({int((fp["m"] > b).sum()) for b in thresholds}) >= 4
         rng = np.random.default_rng(3)
         nnz, n1 = tr.dev.nnz, tr.dev.n_rows
         rows = np.repeat(np.arange(n1), np.diff(tr.dev.pattern()[0]))

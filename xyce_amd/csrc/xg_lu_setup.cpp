@@ -403,11 +403,14 @@ struct CompLu {
 // The limits are also the solution's precision.  A joined child's columns are
 // subtracted group by group from entries of full size; as a front of its own
 // it sums them from zero and adds the sum once.  On power grids, whose rows
-// nearly cancel, eight columns up to 64 rows instead of 24 took 1.2 times the
-// error (28 x 28 mesh: 1.7e-15 against 1.35e-15; no joining at all: 1.26e-15 with
-// one chain per entry).  5,000-gate logic: 18,215 fronts in 26 levels without,
-// 5 levels with; 100 x 100 grid 34 levels and 6, 10,000-node ladder 23 and 4.
-constexpr int64_t kMergeRows = 64, kMergeSmallRows = 24, kMergeSmall = 8, kMergeBig = 16,
+// nearly cancel, eight columns up to 64 rows instead of 25 cost 1.2 times the
+// error (28 x 28 mesh: 1.68e-15 against 1.30e-15; no joining and one chain per
+// entry: 1.26e-15).  Milliseconds per solve of the 100 x 100 and the 500 x 500 grid
+// and the 10,000-node ladder: 1.60 10.4 0.234; at 64 rows and 24 columns 1.64
+// 10.8 0.243; at 20 rows 1.86 11.4 0.288, at 16 columns 1.60 11.2 0.235.
+// 5,000-gate logic: 18,215 fronts in 26 levels without, 5 levels with;
+// 100 x 100 grid 34 levels and 6, 10,000-node ladder 23 and 4.
+constexpr int64_t kMergeRows = 64, kMergeSmallRows = 25, kMergeSmall = 8, kMergeBig = 20,
                   kMergeFlops = 30000000;
 
 std::vector<std::vector<int32_t>> front_tree(int32_t n, const std::vector<int32_t> &parent,
