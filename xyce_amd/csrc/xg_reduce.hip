@@ -87,11 +87,13 @@ __device__ __forceinline__ double fold(double acc, const int32_t *__restrict__ s
 }
 
 // The 64 lanes' sums added to r in lane order; each read with readlane (the
-// reads do not wait on the additions, so only the adds are serial).
+// reads do not wait on the additions, so only the adds are serial), kAhead of
+// them at a time: each takes two scalar registers.
+template <int kAhead>
 __device__ __forceinline__ double add_lanes(double r, double acc) {
   const long long bits = __double_as_longlong(acc);
   const int lo = (int)bits, hi = (int)(bits >> 32);
-#pragma unroll 16
+#pragma unroll kAhead
   for (int l = 0; l < 64; ++l) {
     const unsigned a = (unsigned)__builtin_amdgcn_readlane(lo, l);
     const long long h = (long long)__builtin_amdgcn_readlane(hi, l);
@@ -133,7 +135,7 @@ __device__ __forceinline__ void fold_wide(const ReduceBatch &b, int w,
     for (int u = 0; u < kPiece; ++u) acc = acc + v[u];
   }
   double *out = b.out[k];
-  const double r = add_lanes(b.overwrite ? 0.0 : out[t], acc);
+  const double r = add_lanes<16>(b.overwrite ? 0.0 : out[t], acc);
   if (lane == 0) out[t] = r;
 }
 
@@ -246,7 +248,7 @@ __global__ void __launch_bounds__(kBlock)
   for (int32_t c = rb; c < re; ++c) acc = acc + b.partial[p.pbase + c];
   double *out = b.out[k];
   double r = b.overwrite ? 0.0 : out[t];
-  r = add_lanes(r, acc);  // lane runs in lane order
+  r = add_lanes<64>(r, acc);  // lane runs in lane order (16 at a time: 0.6 us more)
   if (lane == 0) out[t] = r;
 }
 
